@@ -23,6 +23,7 @@
 #include "ill_pass.h"
 #include "ill_gemv.h"
 #include "ill_ops.h"
+#include "ill_rows.h"
 #include "ill_quant.h"
 #include "ill_ildraft_host.h"
 #include "ill_tok.h"
@@ -165,7 +166,8 @@ struct ill_engine {
   OpLayerW* dolayers = nullptr;
   std::vector<OpLayerW> holayers;
   OpCtx octx{};
-  float* opart = nullptr;   // split-K partials of the layer-by-layer GEMMs
+  float* opart = nullptr;   // split-K partials of the layer-by-layer GEMMs; row kernels: attention states
+  float* ssq = nullptr;     // [ILL_OP_MAXM][ROW_SSQ] sum-of-squares partials of the row kernels
   int q8g = 64;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;   // bracket the last single-pass launch
 };
@@ -419,10 +421,43 @@ bool op_gemm(ill_engine* e, const __half* A, const OpMat& W, int M, int layer, f
   return false;
 }
 
+// The kernels of one pass of up to 16 rows of a q8 or f16 model (ill_rows.h); MT: the rows a
+// workgroup holds.
+template <int FMT, int MT>
+void row_seq(ill_engine* e, int M, int lm_rows) {
+  const OpCtx& c = e->octx;
+  hipStream_t s = e->stream;
+  hipLaunchKernelGGL(row_embed_kernel<FMT>, dim3((M + 3) / 4), dim3(256), 0, s, c, e->ssq, M);
+  // one attention workgroup per (row, KV group) and 512 positions of the context the host
+  // expects (the result does not depend on the split)
+  const int nch = (e->pos_hint + M + 63) / 64;
+  const int nsplit = std::max(1, std::min(ROW_NSPLIT, (nch + 7) / 8));
+  for (int l = 0; l < e->layers; l++) {
+    const OpLayerW& L = e->holayers[l];
+    hipLaunchKernelGGL((row_qkv_kernel<FMT, MT>), dim3(ILL_NQB), dim3(448), 0, s, c, L.qkv, L.ln1, L.bqkv, e->ssq, l, M, e->pos_hint);
+    hipLaunchKernelGGL(row_attn_kernel, dim3(M * ILL_NKV * nsplit), dim3(64 * ILL_WAVES), 0, s, c, l, M, nsplit, e->opart);
+    hipLaunchKernelGGL((row_o_kernel<FMT, MT>), dim3(ILL_NOT), dim3(448), 0, s, c, L.o, e->opart, e->ssq, M, nsplit);
+    hipLaunchKernelGGL((row_gu_kernel<FMT, MT>), dim3(2 * ILL_FF / 64), dim3(512), 0, s, c, L.gu, L.ln2, e->ssq, M);
+    hipLaunchKernelGGL((row_down_kernel<FMT, MT>), dim3(ILL_NOT), dim3(1024), 0, s, c, L.d, e->ssq, M);
+  }
+  if (lm_rows > 0) {
+    hipLaunchKernelGGL(op_norm_kernel, dim3((lm_rows + 3) / 4), dim3(256), 0, s, c, c.fnorm, M - lm_rows, lm_rows);
+    op_gemm<FMT, OP_LMH>(e, c.xn, c.emb, lm_rows, 0, nullptr);
+  }
+  hipLaunchKernelGGL(op_commit_kernel, dim3(1), dim3(ILL_WG_THREADS), 0, s, e->args, (const uint64_t*)c.amax, e->vocab / OP_BN, c.kvswz);
+}
+
 // The kernels of one pass over M rows (control block and State already written): layers,
 // lm_head on the last lm_rows rows (0: none), commit.
 template <int FMT>
 void op_seq(ill_engine* e, int M, int lm_rows) {
+  if constexpr (FMT != 2)
+    if (M <= 16) {
+      if (M == 1) row_seq<FMT, 1>(e, M, lm_rows);
+      else if (M <= 4) row_seq<FMT, 4>(e, M, lm_rows);
+      else row_seq<FMT, 16>(e, M, lm_rows);
+      return;
+    }
   const OpCtx& c = e->octx;
   hipStream_t s = e->stream;
   // the embedding with layer 0's RMSNorm (one launch)
@@ -793,7 +828,8 @@ int ill_create(const char* path, int max_context, int max_pass, int max_steps, i
   ok = ok && dalloc((void**)&e->dolayers, sizeof(OpLayerW) * layers) && dalloc((void**)&e->octx.x, (size_t)ILL_OP_MAXM * ILL_H * 4) &&
        dalloc((void**)&e->octx.xn, (size_t)ILL_OP_MAXM * ILL_H * 2) && dalloc((void**)&e->octx.q, (size_t)ILL_OP_MAXM * ILL_H * 4) &&
        dalloc((void**)&e->octx.ao, (size_t)ILL_OP_MAXM * ILL_H * 2) && dalloc((void**)&e->octx.h, (size_t)ILL_OP_MAXM * ILL_FF * 2) &&
-       dalloc((void**)&e->octx.amax, (size_t)(vocab / OP_BN) * 16 * 8) && dalloc((void**)&e->opart, ILL_OP_PART_BYTES);
+       dalloc((void**)&e->octx.amax, (size_t)(vocab / OP_BN) * 16 * 8) && dalloc((void**)&e->opart, ILL_OP_PART_BYTES) &&
+       dalloc((void**)&e->ssq, (size_t)ILL_OP_MAXM * ROW_SSQ * 4);
   if (!ok) return cleanup(fail(ILL_E_HIP, "device buffer allocation failed"));
   if (hipMemcpy(e->dolayers, e->holayers.data(), sizeof(OpLayerW) * layers, hipMemcpyHostToDevice) != hipSuccess)
     return cleanup(fail(ILL_E_HIP, "layer table upload failed"));
@@ -883,7 +919,7 @@ int ill_destroy(ill_engine* e) {
   if (e->graph) hipGraphDestroy(e->graph);
   void* bufs[] = {e->dweights, e->dlayers, e->st, e->ctl, e->ptoks, e->tree, e->rope, e->kc, e->vt, e->acc,
                   e->lmp, e->pub, e->part, e->logits, e->out_dev, e->args.trace, e->oweights, e->dolayers, e->octx.x, e->octx.xn,
-                  e->octx.q, e->octx.ao, e->octx.h, e->octx.amax, e->opart, e->dtab, e->dtflg, e->dreq};
+                  e->octx.q, e->octx.ao, e->octx.h, e->octx.amax, e->opart, e->ssq, e->dtab, e->dtflg, e->dreq};
   for (void* p : bufs)
     if (p) hipFree(p);
   if (e->out_host) hipHostFree(e->out_host);

@@ -1,0 +1,84 @@
+"""The row kernels (passes of up to 16 rows of the layer-by-layer path) where they can go
+wrong: contexts at the edges of a 64-position chunk, of the 512 positions an attention
+workgroup covers, and of the 4096 positions after which a wave takes a second chunk; passes
+of 1, 3 and 16 rows (the three instantiations) that cross those edges; and a captured step
+replayed where more attention splits are in use than it was captured for. Logits against the
+fp32 oracle (relative L2 <= 1e-2, the activations' f16 rounding), rows of one pass against
+single-row passes bit for bit."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from instantllm_amd import synth, illfile as F
+from oracle import illread, qwen, metrics
+
+pytestmark = pytest.mark.gpu
+
+REL_L2_TOL = 1e-2
+VOCAB = 1024
+NO_EOS = (-5, -5)
+CTX = 4096 + 64
+
+
+@pytest.fixture(scope="module", params=[(F.FMT_Q8, 32), (F.FMT_F16, 64)], ids=["q8g32", "f16"])
+def model(request, tmp_path_factory):
+    from instantllm_amd.engine import Engine
+    fmt, group = request.param
+    path = str(tmp_path_factory.mktemp(f"rows{fmt}") / "m.ill")
+    synth.build_model(path, fmt, seed=6, shape=synth.ModelShape(layers=2, vocab=VOCAB), q8_group=group)
+    m = qwen.Model(illread.load(path))
+    e = Engine(path, max_context=CTX + 64, max_pass=16, max_steps=64)
+    toks = [int(t) for t in np.random.default_rng(600 + fmt).integers(0, VOCAB, size=CTX)]
+    e.set_state(pos=0, n=CTX, maxsteps=64, eos=NO_EOS)
+    e.prefill(toks)
+    yield e, m, toks, e.kv_copy_out(CTX)
+    e.close()
+
+
+def one(e, pos, tok):
+    e.set_state(pos=pos, n=1, maxsteps=64, eos=NO_EOS)
+    e.prefill([tok], write_logits=True)
+    return e.read_logits(0).view(np.uint32)
+
+
+@pytest.mark.parametrize("pos", [0, 55, 504, 511, 1016, 4088])
+@pytest.mark.parametrize("rows", [3, 16])
+def test_pass_rows_equal_single_rows(model, pos, rows):
+    e, m, toks, (k, v) = model
+    chain = toks[pos:pos + rows]
+    singles = [one(e, pos + i, t) for i, t in enumerate(chain)]
+    e.kv_copy_in(k, v)
+    e.set_state(pos=pos, n=rows, maxsteps=64, eos=NO_EOS)
+    e.verify_pass(rows, toks=chain, write_logits=True)
+    for i in range(rows):
+        assert np.array_equal(e.read_logits(i).view(np.uint32), singles[i]), (pos, rows, i)
+    e.kv_copy_in(k, v)
+
+
+@pytest.mark.parametrize("pos", [0, 63, 64, 511, 512, 4095, 4097])
+def test_single_row_matches_oracle(model, pos):
+    e, m, toks, (k, v) = model
+    got = one(e, pos, toks[pos]).view(np.float32)
+    e.kv_copy_in(k, v)
+    cache = m.new_cache(pos + 2)
+    ref = m.forward(toks[:pos + 1], cache)
+    assert metrics.rel_l2(got, ref) <= REL_L2_TOL, pos
+
+
+def test_captured_step_replayed_at_a_longer_context(model):
+    e, m, toks, (k, v) = model
+    e.set_state(pos=20, n=1, maxsteps=64, eos=NO_EOS)
+    e.capture_steps(2)   # captured for one attention split
+    for pos in (511, 1500, 4090):
+        e.set_state(pos=pos, n=1, maxsteps=64, eos=NO_EOS)
+        e.prefill([toks[pos]])
+        for _ in range(2):   # two replays of two steps
+            e.launch_graph(write_logits=True)
+            e.sync()
+        graph = e.read_logits(0).view(np.uint32)
+        committed = [int(t) for t in e.out_tokens()[:5]]
+        for i, t in enumerate([toks[pos]] + committed[:4]):
+            last = one(e, pos + i, t)
+        assert np.array_equal(last, graph), pos
+        e.kv_copy_in(k, v)
