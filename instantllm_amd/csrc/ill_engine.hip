@@ -17,6 +17,8 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "../../include/ill_hip.h"
@@ -310,207 +312,143 @@ int write_pos_n(ill_engine* e, int pos, int n) {
 }
 
 // ---- layer-by-layer path -----------------------------------------------------------------
-// Passes of up to 16 rows: the GEMMs that are not register-direct GEMVs (the lm_head, and the
-// gate/up GEMM with K split) run on the LDS-ring GEMM for q8 and f16, on op_gemm_kernel for
-// q4. q8 dequantizes its weights as they leave the ring instead of into an LDS tile: q8
-// decode after 512 positions 892 -> 859 us, at 4096 1,004 -> 975 us (the lm_head alone
-// 4 us of it). f16 takes a ring of 4 stages here (with the prefill gate/up's 2 it was 14 us
-// slower than op_gemm_kernel; with 4, 873 -> 855 us, at 4096 991 -> 973 us).
-#define OP_SMALL_RING(FMT) ((FMT) != 2)
-#ifndef OP_RING_ST_SMALL_F16
-#define OP_RING_ST_SMALL_F16 4
-#endif
-#define OP_RING_ST_SMALL(FMT, EPI) ((FMT) == 0 ? OP_RING_ST_SMALL_F16 : OP_RING_ST(FMT, EPI))
 #define ILL_OP_PART_BYTES (16u << 20)   // >= slices x rows x N x 4 of every split GEMM
-#define ILL_OP_PART_SPLIT (2u << 20)    // floats: passes of up to 16 rows keep the gate/up
-                                        // partials below, the down GEMM's above
 
-// Returns true when it also wrote the RMSNorm of the updated residual (rows >= norm_row0,
-// weights norm_gamma) into xn: residual GEMMs of passes of up to 16 rows with K split.
-// Passes of up to 16 rows only: a gate/up GEMM given silu_out leaves its K-slice partials
-// in opart for the down GEMM and stores their count there (0: it applied SiLU itself); a
-// residual GEMM given silu_S > 0 takes its A operand from those partials.
-template <int FMT, int EPI>
-bool op_gemm(ill_engine* e, const __half* A, const OpMat& W, int M, int layer, float* resid,
-             const float* norm_gamma = nullptr, int norm_row0 = 0, int* silu_out = nullptr, int silu_S = 0) {
-  OpGemmArgs g;
+OpGemmArgs op_args(ill_engine* e, const __half* A, const OpMat& W, int M, int layer) {
+  OpGemmArgs g{};
   g.c = e->octx;
   g.A = A;
   g.W = W;
   g.M = M;
   g.layer = layer;
-  g.resid = resid;
+  g.resid = e->octx.x;
   g.part = e->opart;
+  g.ksteps = W.K / OP_BK;
   g.pos_hint = e->pos_hint;
-  const int nsteps = W.K / OP_BK, ntn = W.N / OP_BN;
-  if constexpr (EPI != OP_LMH) {
-    if (M > 16) {   // prefill chunk: 64-row tiles, K split only where the tiles are few
-      if (EPI == OP_QKV) {
-        // QKV: 16-row tiles over the whole K and the epilogue in the GEMM (no partials and no
-        // reduction kernel): 512 rows, f16, 13.9 us against 9.7 + 5.4 us split three ways
-        g.ksteps = nsteps;
-        if constexpr (FMT != 2)   // q8 / f16: 32-row tiles streamed through the LDS ring
-          hipLaunchKernelGGL((op_gemm_ring_kernel<FMT, 32, EPI, OP_RING_ST(FMT, EPI)>), dim3(ntn, (M + 31) / 32, 1), dim3(256), 0,
-                             e->stream, g);
-        else
-          hipLaunchKernelGGL((op_gemm_kernel<FMT, 16, EPI, 4>), dim3(ntn, (M + 15) / 16, 1), dim3(256), 0, e->stream, g);
-        return false;
-      }
-      const int mt = (M + 63) / 64;
-      const int cap = (int)(ILL_OP_PART_BYTES / ((size_t)M * W.N * 4));   // partial buffer
-      int S = std::max(1, std::min(std::min(std::min(256 / (ntn * mt), nsteps / 4), OP_MAXS), cap));
-      g.ksteps = (nsteps + S - 1) / S;
-      S = (nsteps + g.ksteps - 1) / g.ksteps;
-      // the many-tile gate/up GEMM streams best with the one-step kernel (more per CU)
-      if constexpr (FMT != 2)
-        hipLaunchKernelGGL((op_gemm_ring_kernel<FMT, 64, EPI, OP_RING_ST(FMT, EPI)>), dim3(ntn, mt, S), dim3(256), 0, e->stream, g);
-      else
-        hipLaunchKernelGGL((op_gemm_kernel<FMT, 64, EPI, EPI == OP_SILU ? 1 : 4>), dim3(ntn, mt, S), dim3(256), 0, e->stream, g);
-      if (S > 1) {
-        if (EPI == OP_RESID && norm_gamma && W.N == ILL_H) {
-          hipLaunchKernelGGL(op_epi_norm_kernel, dim3(M), dim3(ILL_H), 0, e->stream, g, S, norm_gamma, norm_row0);
-          return true;
-        }
-        const int per = EPI == OP_RESID ? W.N : W.N / 2;
-        hipLaunchKernelGGL((op_epi_kernel<EPI>), dim3((M * per + 255) / 256), dim3(256), 0, e->stream, g, S);
-      }
-      return false;
-    }
-  }
-  // up to 16 rows: split K so that about 256 workgroups stream the weights,
-  // at least four k-steps per slice (the split depends on the matrix only, so 1-row and
-  // 16-row passes sum the same partials in the same order)
-  int S = 1;
-  // (QKV of q8 / f16: K not split across workgroups; 36 two-wave workgroups, each wave half
-  // of K, apply the epilogue themselves)
-  constexpr bool QKV1 = EPI == OP_QKV && FMT != 2;
-  if (EPI != OP_LMH && !QKV1) S = std::max(1, std::min(std::min((256 + ntn - 1) / ntn, nsteps / 4), OP_MAXS));
-  g.ksteps = (nsteps + S - 1) / S;
-  S = (nsteps + g.ksteps - 1) / g.ksteps;
-  if (g.ksteps * OP_BK > OP_SMAXK) {
-    fail(ILL_E_ARG, "K slice of %d columns exceeds %d", g.ksteps * OP_BK, OP_SMAXK);
-    return false;
-  }
-  const dim3 grid(ntn, 1, S);
-  if (EPI == OP_RESID && silu_S > 0) {   // A = SwiGLU of the gate/up partials left in opart
-    g.apart = e->opart;
-    g.aS = silu_S;
-    g.part = e->opart + ILL_OP_PART_SPLIT;
-    hipLaunchKernelGGL((op_gemv_kernel<FMT, EPI, true>), grid, dim3(256), 0, e->stream, g);
-  } else if constexpr (QKV1) {
-    hipLaunchKernelGGL((op_gemv_kernel<FMT, EPI, false, 2>), dim3(W.N / 32), dim3(128), 0, e->stream, g);
-  } else if constexpr (OP_SMALL_RING(FMT)) {
-    hipLaunchKernelGGL((op_gemm_ring_kernel<FMT, 16, EPI, OP_RING_ST_SMALL(FMT, EPI)>), grid, dim3(256), 0, e->stream, g);
-  } else {
-    hipLaunchKernelGGL((op_gemm_kernel<FMT, 16, EPI, 4>), grid, dim3(256), 0, e->stream, g);
-  }
-  if constexpr (EPI != OP_LMH) {
-    if (S > 1) {
-      if (EPI == OP_SILU && silu_out && (size_t)S * M * W.N * 4 <= ILL_OP_PART_SPLIT * 4) {
-        *silu_out = S;   // the down GEMM takes the partials
-        return false;
-      }
-      if (EPI == OP_RESID && norm_gamma && W.N == ILL_H) {
-        hipLaunchKernelGGL(op_epi_norm_kernel, dim3(M), dim3(ILL_H), 0, e->stream, g, S, norm_gamma, norm_row0);
-        return true;
-      }
-      const int per = EPI == OP_RESID ? W.N : W.N / 2;
-      hipLaunchKernelGGL((op_epi_kernel<EPI>), dim3((M * per + 255) / 256), dim3(256), 0, e->stream, g, S);
-    }
-  }
-  return false;
+  return g;
 }
 
-// The kernels of one pass of up to 16 rows of a q8 or f16 model (ill_rows.h); MT: the rows a
-// workgroup holds.
+// One product of a prompt chunk (more than ROW_MAXM rows) on the LDS-ring GEMM: 64-row tiles,
+// K split only where the tiles are few. Returns true when it also wrote the RMSNorm (weights
+// norm_gamma) of the updated residual into xn: residual products with K split.
+template <int FMT, int EPI>
+bool op_gemm(ill_engine* e, const __half* A, const OpMat& W, int M, int layer, const float* norm_gamma = nullptr) {
+  OpGemmArgs g = op_args(e, A, W, M, layer);
+  const int nsteps = g.ksteps, ntn = W.N / OP_BN;
+  if constexpr (EPI == OP_QKV) {
+    // 32-row tiles over the whole K and the epilogue in the GEMM (no partials and no reduction
+    // kernel): 512 rows, f16, 13.9 us against 9.7 + 5.4 us split three ways
+    hipLaunchKernelGGL((op_gemm_ring_kernel<FMT, 32, EPI, OP_RING_ST(FMT, EPI)>), dim3(ntn, (M + 31) / 32, 1), dim3(256), 0, e->stream, g);
+    return false;
+  }
+  const int mt = (M + 63) / 64;
+  int S = 1;
+  if constexpr (EPI == OP_RESID) {
+    const int cap = (int)(ILL_OP_PART_BYTES / ((size_t)M * W.N * 4));   // partial buffer
+    S = std::max(1, std::min(std::min(std::min(256 / (ntn * mt), nsteps / 4), OP_MAXS), cap));
+    g.ksteps = (nsteps + S - 1) / S;
+    S = (nsteps + g.ksteps - 1) / g.ksteps;
+  }
+  hipLaunchKernelGGL((op_gemm_ring_kernel<FMT, 64, EPI, OP_RING_ST(FMT, EPI)>), dim3(ntn, mt, S), dim3(256), 0, e->stream, g);
+  if (S == 1) return false;
+  hipLaunchKernelGGL(op_epi_norm_kernel, dim3(M), dim3(ILL_H), 0, e->stream, g, S, norm_gamma, 0);
+  return true;
+}
+
+// The final norm of rows row0 .. row0 + n - 1 (n <= 16) of c.x, the lm_head and its argmax tiles.
+template <int FMT>
+void op_head(ill_engine* e, const OpCtx& c, int row0, int n) {
+  hipLaunchKernelGGL(op_norm_kernel, dim3((n + 3) / 4), dim3(256), 0, e->stream, c, c.fnorm, row0, n);
+  const OpGemmArgs g = op_args(e, e->octx.xn, c.emb, n, 0);
+  // (f16: with the prefill gate/up's 2 stages a 1-row step was 14 us slower than with 4)
+  constexpr int ST = FMT == 0 ? 4 : OP_RING_ST(FMT, OP_LMH);
+  hipLaunchKernelGGL((op_gemm_ring_kernel<FMT, 16, OP_LMH, ST>), dim3(c.emb.N / OP_BN, 1, 1), dim3(256), 0, e->stream, g);
+}
+
+// Attention over a prompt chunk's 16-row blocks blk0 .. (every query head).
+template <int FMT>
+void op_attn_rows(ill_engine* e, int layer, int M, int blk0) {
+  hipLaunchKernelGGL(op_attn_rows_kernel<FMT != 2>, dim3((M + 15) / 16 - blk0, ILL_NH), dim3(64 * OP_RW), 0, e->stream, e->octx, layer, M, blk0);
+}
+
+// The last layer of a prompt chunk after its QKV product. Only the chunk's last row goes on to
+// the lm_head (lm_rows 1) or none does (0): attention for the last row's block, then the
+// row kernels on that row alone. (All 512 rows: about 60 us more per prefill.)
+template <int FMT>
+void op_last_row(ill_engine* e, int M, int lm_rows) {
+  if (lm_rows == 0) return;
+  hipStream_t s = e->stream;
+  const int l = e->layers - 1;
+  const OpLayerW& L = e->holayers[l];
+  OpCtx c = e->octx;
+  c.x += (size_t)(M - 1) * ILL_H;
+  c.ao += (size_t)(M - 1) * ILL_H;
+  op_attn_rows<FMT>(e, l, M, (M + 15) / 16 - 1);
+  hipLaunchKernelGGL((row_o_kernel<FMT, 1, true>), dim3(ILL_NOT), dim3(448), 0, s, c, L.o, nullptr, e->ssq, 1, 0);
+  hipLaunchKernelGGL((row_gu_kernel<FMT, 1>), dim3(2 * ILL_FF / 64), dim3(512), 0, s, c, L.gu, L.ln2, e->ssq, 1);
+  hipLaunchKernelGGL((row_down_kernel<FMT, 1>), dim3(ILL_NOT), dim3(1024), 0, s, c, L.d, e->ssq, 1);
+  op_head<FMT>(e, c, 0, 1);
+}
+
+// The layers (and lm_head) of a pass on the row kernels (ill_rows.h), MT rows per workgroup.
+// Up to 16 rows: any pass of a q8 or f16 model. More (at most ROW_MAXM): a prompt chunk.
 template <int FMT, int MT>
 void row_seq(ill_engine* e, int M, int lm_rows) {
   const OpCtx& c = e->octx;
   hipStream_t s = e->stream;
+  const int mg = (M + 15) / 16;
   hipLaunchKernelGGL(row_embed_kernel<FMT>, dim3((M + 3) / 4), dim3(256), 0, s, c, e->ssq, M);
-  // one attention workgroup per (row, KV group) and 512 positions of the context the host
-  // expects (the result does not depend on the split)
+  // up to 16 rows: one attention workgroup per (row, KV group) and 512 positions of the context
+  // the host expects (the result does not depend on the split)
   const int nch = (e->pos_hint + M + 63) / 64;
   const int nsplit = std::max(1, std::min(ROW_NSPLIT, (nch + 7) / 8));
   for (int l = 0; l < e->layers; l++) {
     const OpLayerW& L = e->holayers[l];
-    hipLaunchKernelGGL((row_qkv_kernel<FMT, MT>), dim3(ILL_NQB), dim3(448), 0, s, c, L.qkv, L.ln1, L.bqkv, e->ssq, l, M, e->pos_hint);
-    hipLaunchKernelGGL(row_attn_kernel, dim3(M * ILL_NKV * nsplit), dim3(64 * ILL_WAVES), 0, s, c, l, M, nsplit, e->opart);
-    hipLaunchKernelGGL((row_o_kernel<FMT, MT>), dim3(ILL_NOT), dim3(448), 0, s, c, L.o, e->opart, e->ssq, M, nsplit);
-    hipLaunchKernelGGL((row_gu_kernel<FMT, MT>), dim3(2 * ILL_FF / 64), dim3(512), 0, s, c, L.gu, L.ln2, e->ssq, M);
-    hipLaunchKernelGGL((row_down_kernel<FMT, MT>), dim3(ILL_NOT), dim3(1024), 0, s, c, L.d, e->ssq, M);
+    hipLaunchKernelGGL((row_qkv_kernel<FMT, MT>), dim3(ILL_NQB, mg), dim3(448), 0, s, c, L.qkv, L.ln1, L.bqkv, e->ssq, l, M, e->pos_hint);
+    if (M > 16) {
+      if (l + 1 == e->layers) return op_last_row<FMT>(e, M, lm_rows);
+      op_attn_rows<FMT>(e, l, M, 0);
+      if constexpr (MT == 16) hipLaunchKernelGGL((row_o_kernel<FMT, MT, true>), dim3(ILL_NOT, mg), dim3(448), 0, s, c, L.o, nullptr, e->ssq, M, 0);
+    } else {
+      hipLaunchKernelGGL(row_attn_kernel<FMT != 2>, dim3(M * ILL_NKV * nsplit), dim3(64 * ILL_WAVES), 0, s, c, l, M, nsplit, e->opart);
+      hipLaunchKernelGGL((row_o_kernel<FMT, MT, false>), dim3(ILL_NOT), dim3(448), 0, s, c, L.o, e->opart, e->ssq, M, nsplit);
+    }
+    hipLaunchKernelGGL((row_gu_kernel<FMT, MT>), dim3(2 * ILL_FF / 64, mg), dim3(512), 0, s, c, L.gu, L.ln2, e->ssq, M);
+    hipLaunchKernelGGL((row_down_kernel<FMT, MT>), dim3(ILL_NOT, mg), dim3(1024), 0, s, c, L.d, e->ssq, M);
   }
-  if (lm_rows > 0) {
-    hipLaunchKernelGGL(op_norm_kernel, dim3((lm_rows + 3) / 4), dim3(256), 0, s, c, c.fnorm, M - lm_rows, lm_rows);
-    op_gemm<FMT, OP_LMH>(e, c.xn, c.emb, lm_rows, 0, nullptr);
-  }
-  hipLaunchKernelGGL(op_commit_kernel, dim3(1), dim3(ILL_WG_THREADS), 0, s, e->args, (const uint64_t*)c.amax, e->vocab / OP_BN, c.kvswz);
+  if (lm_rows > 0) op_head<FMT>(e, c, M - lm_rows, lm_rows);
 }
 
-// The kernels of one pass over M rows (control block and State already written): layers,
-// lm_head on the last lm_rows rows (0: none), commit.
+// The layers (and lm_head) of a prompt chunk on the ring GEMMs.
 template <int FMT>
-void op_seq(ill_engine* e, int M, int lm_rows) {
-  if constexpr (FMT != 2)
-    if (M <= 16) {
-      if (M == 1) row_seq<FMT, 1>(e, M, lm_rows);
-      else if (M <= 4) row_seq<FMT, 4>(e, M, lm_rows);
-      else row_seq<FMT, 16>(e, M, lm_rows);
-      return;
-    }
+void chunk_seq(ill_engine* e, int M, int lm_rows) {
   const OpCtx& c = e->octx;
   hipStream_t s = e->stream;
   // the embedding with layer 0's RMSNorm (one launch)
   hipLaunchKernelGGL(op_embed_norm_kernel<FMT>, dim3((M + 3) / 4), dim3(256), 0, s, c, e->holayers[0].ln1, M);
-  // passes of up to 16 rows: attention split over up to 8 workgroups per (row, head), one
-  // per 1024 positions of context (the result does not depend on the split)
-  const int nch = (e->pos_hint + M + 63) / 64;
-  const int nsplit = std::max(1, std::min(OP_NSPLIT, (nch + 15) / 16));
-  // passes of up to 16 rows (q8 / f16; q4 ones run on the pass kernel): the O projection
-  // runs per head inside the attention kernel (one split) or the split combine, always with
-  // the same arithmetic, so the split does not change the result
-  const bool ofuse = FMT != 2 && M <= 16;
-  float* opart_o = e->opart + ILL_OP_PART_SPLIT;   // [head][row][896] O partials
-  // each residual update also writes the next RMSNorm where its K is split (op_gemm returns
-  // whether it did)
-  bool normed = true;   // (layer 0's came with the embedding)
+  auto norm = [&](const float* gamma) { hipLaunchKernelGGL(op_norm_kernel, dim3((M + 3) / 4), dim3(256), 0, s, c, gamma, 0, M); };
+  // each residual update also writes the next RMSNorm where its K is split
   for (int l = 0; l < e->layers; l++) {
     const OpLayerW& L = e->holayers[l];
-    if (!normed) hipLaunchKernelGGL(op_norm_kernel, dim3((M + 3) / 4), dim3(256), 0, s, c, L.ln1, 0, M);
-    op_gemm<FMT, OP_QKV>(e, c.xn, L.qkv, M, l, nullptr);
-    if (M > 16) hipLaunchKernelGGL(op_attn_rows_kernel<FMT != 2>, dim3((M + 15) / 16, ILL_NH), dim3(64 * OP_RW), 0, s, c, l, M);
-    else {
-      float* op1 = ofuse && nsplit == 1 ? opart_o : nullptr;
-      hipLaunchKernelGGL(op_attn_kernel<FMT>, dim3(M * ILL_NH * nsplit), dim3(64 * ILL_WAVES), 0, s, c, l, M, nsplit, e->opart,
-                         L.oh, op1);
-      if (nsplit > 1)
-        hipLaunchKernelGGL(op_attn_combine_kernel<FMT>, dim3(M * ILL_NH), dim3(64 * ILL_WAVES), 0, s, c, (const float*)e->opart,
-                           L.oh, ofuse ? opart_o : (float*)nullptr, M);
-      if (ofuse) {   // the residual + norm over the 14 per-head O partials (head order)
-        OpGemmArgs g{};
-        g.c = c;
-        g.W = L.o;
-        g.M = M;
-        g.layer = l;
-        g.resid = c.x;
-        g.part = opart_o;
-        hipLaunchKernelGGL(op_epi_norm_kernel, dim3(M), dim3(ILL_H), 0, s, g, ILL_NH, L.ln2, 0);
-      }
-    }
-    const bool fuse = M <= 16;   // the SwiGLU hand-over (the residual + norm fusion: any M)
-    if (!ofuse && !op_gemm<FMT, OP_RESID>(e, c.ao, L.o, M, l, c.x, L.ln2, 0))
-      hipLaunchKernelGGL(op_norm_kernel, dim3((M + 3) / 4), dim3(256), 0, s, c, L.ln2, 0, M);
-    int silu_S = 0;
-    op_gemm<FMT, OP_SILU>(e, c.xn, L.gu, M, l, nullptr, nullptr, 0, fuse ? &silu_S : nullptr);
-    const bool last = l + 1 == e->layers;
-    const float* next = last ? (lm_rows > 0 ? c.fnorm : nullptr) : e->holayers[l + 1].ln1;
-    normed = op_gemm<FMT, OP_RESID>(e, c.h, L.d, M, l, c.x, next, last ? M - lm_rows : 0, nullptr, silu_S);
+    op_gemm<FMT, OP_QKV>(e, c.xn, L.qkv, M, l);
+    if (l + 1 == e->layers) return op_last_row<FMT>(e, M, lm_rows);
+    op_attn_rows<FMT>(e, l, M, 0);
+    if (!op_gemm<FMT, OP_RESID>(e, c.ao, L.o, M, l, L.ln2)) norm(L.ln2);
+    op_gemm<FMT, OP_SILU>(e, c.xn, L.gu, M, l);
+    const float* next = e->holayers[l + 1].ln1;
+    if (!op_gemm<FMT, OP_RESID>(e, c.h, L.d, M, l, next)) norm(next);
   }
-  if (lm_rows > 0) {
-    if (!normed) hipLaunchKernelGGL(op_norm_kernel, dim3((lm_rows + 3) / 4), dim3(256), 0, s, c, c.fnorm, M - lm_rows, lm_rows);
-    op_gemm<FMT, OP_LMH>(e, c.xn, c.emb, lm_rows, 0, nullptr);
-  }
-  hipLaunchKernelGGL(op_commit_kernel, dim3(1), dim3(ILL_WG_THREADS), 0, s, e->args, (const uint64_t*)c.amax, e->vocab / OP_BN, c.kvswz);
+}
+
+// The kernels of one pass over M rows (control block and State already written): layers,
+// lm_head on the last lm_rows rows (0: none; at most 1 past 16 rows), commit.
+template <int FMT>
+void op_seq(ill_engine* e, int M, int lm_rows) {
+  if (M == 1) row_seq<FMT, 1>(e, M, lm_rows);
+  else if (M <= 4) row_seq<FMT, 4>(e, M, lm_rows);
+  else if (M <= ROW_MAXM) row_seq<FMT, 16>(e, M, lm_rows);
+  else chunk_seq<FMT>(e, M, lm_rows);
+  hipLaunchKernelGGL(op_commit_kernel, dim3(1), dim3(ILL_WG_THREADS), 0, e->stream, e->args, (const uint64_t*)e->octx.amax, e->vocab / OP_BN, e->octx.kvswz);
 }
 
 void op_seq_fmt(ill_engine* e, int M, int lm_rows) {
@@ -712,7 +650,7 @@ int ill_create(const char* path, int max_context, int max_pass, int max_steps, i
     w.wd = D + L.dW; w.sd = (const uint32_t*)(D + L.dS);
     w.bqkv = (const float*)(D + L.b); w.ln1 = (const float*)(D + L.ln1); w.ln2 = (const float*)(D + L.ln2);
   }
-  // ---- layer-by-layer path: the .ill matrices as stored (row-major, file row orders)
+  // ---- layer-by-layer path: the .ill matrices (file row orders) tiled for its kernels
   {
     std::vector<size_t> place(count, 0);
     size_t otot = 0;
@@ -720,65 +658,64 @@ int ill_create(const char* path, int max_context, int max_pass, int max_steps, i
       place[id] = otot;
       otot += al256(size(id));
     }
-    // q8 / f16: W_o head-major for the attention-fused O projection (OpLayerW::oh)
-    const bool ohead = fmt != 2;
-    const int es = fmt == 0 ? 2 : 1, nchk = 64 * es / 16, qg = e->q8g;
-    const size_t ohw = (size_t)ILL_NH * nchk * ILL_H * 16, ohs = (size_t)ILL_NH * ILL_H * 4;
-    std::vector<size_t> p_ohw(layers, 0), p_ohs(layers, 0);
-    if (ohead)
-      for (int l = 0; l < layers; l++) {
-        p_ohw[l] = otot;
-        otot += al256(ohw);
-        p_ohs[l] = otot;
-        otot += al256(ohs);
-      }
+    const int qg = e->q8g;
     std::vector<uint8_t> oh(otot);
     for (int id = 0; id < count; id++)
       if (size(id)) memcpy(oh.data() + place[id], base + off(id), size(id));
-    // q8 / f16: the matrices tiled for the GEMM kernels (op_wt_off / op_st_off, ill_ops.h)
-    auto tile = [&](int idw, int ids, int N, int K) {
-      const int es = fmt == 0 ? 2 : 1, unit = 16 / es;
-      if (N % 128 || K % 64 || size(idw) < (size_t)N * K * es || (fmt == 1 && size(ids) < (size_t)N * (K / qg) * 2)) return false;
+    // (op_wt_off, op_w4_off, op_st_off of ill_ops.h); 128-row blocks dealt to a few threads
+    auto tile_rows = [&](int idw, int ids, int K, int r0, int r1) {
       const uint8_t* src = base + off(idw);
       uint8_t* dst = oh.data() + place[idw];
-      for (int r = 0; r < N; r++)
+      if (fmt == 2) {
+        const uint32_t* ss = (const uint32_t*)(base + off(ids));
+        uint32_t* sd = (uint32_t*)(oh.data() + place[ids]);
+        auto evens = [](uint32_t v) {   // nibbles 0, 2, 4, 6 into the low half
+          v &= 0x0f0f0f0fu;
+          v = (v | (v >> 4)) & 0x00ff00ffu;
+          return (v | (v >> 8)) & 0xffffu;
+        };
+        for (int r = r0; r < r1; r++)
+          for (int k = 0; k < K; k += 8) {
+            uint32_t x;
+            memcpy(&x, src + ((size_t)r * K + k) / 2, 4);   // column k + c in nibble c
+            const uint32_t y = evens(x) | (evens(x >> 4) << 16);
+            memcpy(dst + op_w4_off(r, k, K), &y, 4);
+            if (k % 64 == 0) sd[op_st_off(r, k, K, 64)] = ss[((size_t)r * K + k) / 64];
+          }
+        return;
+      }
+      const int es = fmt == 0 ? 2 : 1, unit = 16 / es;
+      for (int r = r0; r < r1; r++)
         for (int k = 0; k < K; k += unit) memcpy(dst + op_wt_off(r, k, K, es), src + ((size_t)r * K + k) * es, 16);
       if (fmt == 1) {
         const uint16_t* ss = (const uint16_t*)(base + off(ids));
         uint16_t* sd = (uint16_t*)(oh.data() + place[ids]);
-        for (int r = 0; r < N; r++)
+        for (int r = r0; r < r1; r++)
           for (int g = 0; g < K / qg; g++) sd[op_st_off(r, g * qg, K, qg)] = ss[(size_t)r * (K / qg) + g];
       }
-      return true;
     };
-    if (fmt != 2) {
-      bool tiled = tile(0, 1, vocab, ILL_H);
-      for (int l = 0; l < layers && tiled; l++) {
-        const int b = 3 + 12 * l;
-        tiled = tile(b + 1, b + 2, ILL_QKV, ILL_H) && tile(b + 4, b + 5, ILL_H, ILL_H) && tile(b + 7, b + 8, 2 * ILL_FF, ILL_H) &&
-                tile(b + 9, b + 10, ILL_H, ILL_FF);
-      }
-      if (!tiled) return cleanup(fail(ILL_E_FILE, "a q8 / f16 matrix does not have the expected shape"));
+    struct Mat {
+      int idw, ids, N, K;
+    };
+    std::vector<Mat> mats = {{0, 1, vocab, ILL_H}};
+    for (int l = 0; l < layers; l++) {
+      const int b = 3 + 12 * l;
+      mats.insert(mats.end(), {{b + 1, b + 2, ILL_QKV, ILL_H}, {b + 4, b + 5, ILL_H, ILL_H}, {b + 7, b + 8, 2 * ILL_FF, ILL_H}, {b + 9, b + 10, ILL_H, ILL_FF}});
     }
-    if (ohead)
-      for (int l = 0; l < layers; l++) {
-        const int b = 3 + 12 * l;
-        if (size(b + 4) < (size_t)ILL_H * ILL_H * es || (fmt == 1 && size(b + 5) < (size_t)ILL_H * (ILL_H / qg) * 2))
-          return cleanup(fail(ILL_E_FILE, "layer %d: W_o tensors too small", l));
-        const uint8_t* wsrc = base + off(b + 4);
-        const uint16_t* ssrc = (const uint16_t*)(base + off(b + 5));
-        for (int h = 0; h < ILL_NH; h++)
-          for (int i = 0; i < nchk; i++)
-            for (int r = 0; r < ILL_H; r++)
-              memcpy(oh.data() + p_ohw[l] + (((size_t)h * nchk + i) * ILL_H + r) * 16, wsrc + ((size_t)r * ILL_H + 64 * h) * es + 16 * i, 16);
-        if (fmt == 1)
-          for (int h = 0; h < ILL_NH; h++)
-            for (int r = 0; r < ILL_H; r++) {
-              const uint32_t v = (uint32_t)ssrc[(size_t)r * (ILL_H / qg) + (64 * h) / qg] |
-                                 ((uint32_t)ssrc[(size_t)r * (ILL_H / qg) + (64 * h + 32) / qg] << 16);
-              memcpy(oh.data() + p_ohs[l] + ((size_t)h * ILL_H + r) * 4, &v, 4);
-            }
-      }
+    auto tile_part = [&](int part, int parts) {   // every parts-th 128-row block of every matrix
+      for (const Mat& t : mats)
+        for (int r = 128 * part; r < t.N; r += 128 * parts) tile_rows(t.idw, t.ids, t.K, r, r + 128);
+    };
+    const int nth = std::max(1, std::min(8, (int)std::thread::hardware_concurrency()));
+    std::vector<std::thread> th;
+    try {
+      for (int i = 1; i < nth; i++) th.emplace_back(tile_part, i, nth);
+    } catch (const std::system_error&) {   // no more threads: the rest of the parts run here
+    }
+    const int started = (int)th.size() + 1;
+    tile_part(0, nth);
+    for (int i = started; i < nth; i++) tile_part(i, nth);
+    for (auto& t : th) t.join();
     if (hipMalloc(&e->oweights, otot) != hipSuccess) return cleanup(fail(ILL_E_HIP, "weights allocation failed (%zu B)", otot));
     if (hipMemcpy(e->oweights, oh.data(), otot, hipMemcpyHostToDevice) != hipSuccess) return cleanup(fail(ILL_E_HIP, "weights upload failed"));
     uint8_t* O = e->oweights;
@@ -797,11 +734,6 @@ int ill_create(const char* path, int max_context, int max_pass, int max_steps, i
       OpLayerW& w = e->holayers[l];
       w.qkv = mk(b + 1, b + 2, ILL_QKV, ILL_H);
       w.o = mk(b + 4, b + 5, ILL_H, ILL_H);
-      w.oh = w.o;
-      if (ohead) {
-        w.oh.w = O + p_ohw[l];
-        w.oh.s = (const uint16_t*)(O + p_ohs[l]);
-      }
       w.gu = mk(b + 7, b + 8, 2 * ILL_FF, ILL_H);
       w.d = mk(b + 9, b + 10, ILL_H, ILL_FF);
       w.bqkv = (const float*)(O + place[b + 3]);

@@ -28,12 +28,12 @@
 #define ILL_OP_MAXM 512
 
 struct OpMat {
-  const uint8_t* w;    // q4: codes [N][K/2]; q8: int8, f16: halves, both tiled (op_wt_off)
-  const uint16_t* s;   // q4: [N][K/64][2] f16 (scale, min); q8: f16 tiled (op_st_off); f16: unused
+  const uint8_t* w;    // q4 nibbles, q8 int8 or f16 halves, tiled (op_wt_off, op_w4_off)
+  const uint16_t* s;   // q4: f16 (scale, min) pairs, q8: f16 scales, tiled (op_st_off); f16: unused
   int N, K, qg;        // qg: q8 group size (32 or 64)
 };
 
-// The q8 and f16 matrices of the layer-by-layer path are tiled, so that a wave's 16-byte
+// The matrices of the layer-by-layer path are tiled, so that a wave's 16-byte
 // loads of one k-step (64 columns) read whole cache lines: 128-row blocks, k-steps, 16-row
 // sub-tiles of 16 x 64 weights, inside which 16-byte units are ordered (8-column half e,
 // 16-column group kg, row n). Element (r, k) of an N x K matrix of es-byte weights (N a
@@ -41,9 +41,11 @@ struct OpMat {
 //   ((((r >> 7) * (K / 64) + (k >> 6)) * 8 + ((r & 127) >> 4)) * 64 es
 //    + ((e * 4 + kg) * 16 + (r & 15)) * 16 + (k & 7) * es)   with kg = (k & 63) >> 4,
 //   e = (k >> 3) & 1 for f16; for q8 a unit holds 16 columns (e = 0, (k & 15) bytes).
-// A lane (kg, n) of op_fetch_b then reads 1 KB contiguous with its wave, and a thread of
-// op_fetch_w (row, 32 columns) two 256-byte runs. q8 scales: [block][k-step][128 rows]
-// [64 / qg] (op_st_off).
+// A lane (kg, n) then reads 1 KB contiguous with its wave. q8 scales: [block][k-step]
+// [128 rows][64 / qg] (op_st_off). q4: a lane (kg, n)'s 16 columns are two dwords of 8
+// nibbles (512 bytes per sub-tile, op_w4_off), column 2 i + j of the 8 in nibble i + 4 j, so
+// that (word >> 4 i) & 0x000f000f holds two neighbouring columns; (scale, min) pairs
+// [block][k-step][128 rows].
 __host__ __device__ inline size_t op_wt_off(int r, int k, int K, int es) {
   const size_t tile = ((size_t)(r >> 7) * (K >> 6) + (k >> 6)) * 8 + ((r & 127) >> 4);
   const int kg = (k & 63) >> 4;
@@ -55,13 +57,13 @@ __host__ __device__ inline size_t op_st_off(int r, int k, int K, int qg) {
   return (((size_t)(r >> 7) * (K >> 6) + (k >> 6)) * 128 + (r & 127)) * (64 / qg) + ((k & 63) / qg);
 }
 
+__host__ __device__ inline size_t op_w4_off(int r, int k, int K) {   // of the dword with column k
+  const size_t tile = ((size_t)(r >> 7) * (K >> 6) + (k >> 6)) * 8 + ((r & 127) >> 4);
+  return tile * 512 + (size_t)((((k & 63) >> 4) * 16 + (r & 15)) * 8 + ((k >> 3) & 1) * 4);
+}
+
 struct OpLayerW {
   OpMat qkv, o, gu, d;
-  // W_o again, head-major for the O projection folded into attention (q8 / f16): codes
-  // [head][16-byte column chunk][896 rows] (4 chunks q8, 8 f16), scales (q8) [head][896 rows]
-  // as u32 (scale of k 0-31 | scale of k 32-63 << 16), so that a lane per row reads
-  // consecutive 16 bytes
-  OpMat oh;
   const float* bqkv;
   const float* ln1;
   const float* ln2;
@@ -113,9 +115,9 @@ __device__ __forceinline__ int op_depth(const OpCtx& c, int mode, int t) {
 template <int FMT>
 __device__ __forceinline__ float op_dequant1(const OpMat& m, int r, int k) {
   if constexpr (FMT == 2) {
-    const uint8_t b = m.w[(size_t)r * (m.K / 2) + k / 2];
-    const float q = (float)((k & 1) ? (b >> 4) : (b & 15));
-    const uint32_t sm = *(const uint32_t*)(m.s + ((size_t)r * (m.K / 64) + k / 64) * 2);
+    const uint32_t x = *(const uint32_t*)(m.w + op_w4_off(r, k, m.K));
+    const float q = (float)((x >> (4 * (((k & 7) >> 1) + 4 * (k & 1)))) & 15);
+    const uint32_t sm = *((const uint32_t*)m.s + op_st_off(r, k, m.K, 64));
     return h2f(sm & 0xffff) * q + h2f(sm >> 16);
   } else if constexpr (FMT == 1) {
     const float q = (float)(int8_t)m.w[op_wt_off(r, k, m.K, 1)];
@@ -195,42 +197,13 @@ struct OpGemmArgs {
   float* resid;      // OP_RESID: [M][896] += Y
   float* part;       // split K: [slices][M][N] fp32 partials
   int ksteps;        // 64-column steps per K slice
-  const float* apart;   // op_gemv_kernel<.., SILU = true>: gate/up partials [aS][M][2K]
-  int aS;
   int pos_hint;         // the State's pos as the host expects it (QKV epilogue: rotary rows
                         // are loaded for pos_hint + row with the partials)
 };
 
 #define OP_BN 128
 #define OP_BK 64
-#define OP_LDK 72    // LDS row stride in halves (padding against bank conflicts)
 #define OP_MAXS 24   // K slices of a split GEMM at most
-
-// One k-step (64 columns) of the weight tile, rows n0 .. n0+127, as loaded from HBM, and
-// its dequantization into LDS [128][OP_LDK] f16. Thread -> (row tid / 2, half tid % 2).
-template <int FMT>
-struct WRaw {
-  uint4 b[FMT == 2 ? 1 : (FMT == 1 ? 2 : 4)];
-  // q4: (scale, min) pair; q8: the scale, kept 16-bit so that the load needs no widening
-  // (which would wait for it at once)
-  std::conditional_t<FMT == 1, uint16_t, uint32_t> sm;
-};
-
-template <int FMT>
-__device__ __forceinline__ void op_fetch_w(const OpMat& W, int n0, int k0, int tid, WRaw<FMT>& r) {
-  const int row = n0 + (tid >> 1), hf = tid & 1;
-  if constexpr (FMT == 2) {
-    r.b[0] = gld((const uint4*)(W.w + (size_t)row * (W.K / 2) + k0 / 2 + 16 * hf));
-    r.sm = gld((const uint32_t*)(W.s + ((size_t)row * (W.K / 64) + k0 / 64) * 2));
-  } else if constexpr (FMT == 1) {
-    r.b[0] = gld((const uint4*)(W.w + op_wt_off(row, k0 + 32 * hf, W.K, 1)));
-    r.b[1] = gld((const uint4*)(W.w + op_wt_off(row, k0 + 32 * hf + 16, W.K, 1)));
-    r.sm = gld(W.s + op_st_off(row, k0 + 32 * hf, W.K, W.qg));
-  } else {
-#pragma unroll
-    for (int i = 0; i < 4; i++) r.b[i] = gld((const uint4*)(W.w + op_wt_off(row, k0 + 32 * hf + 8 * i, W.K, 2)));
-  }
-}
 
 // q8 dequantization, 4 weights at a time: s * (f16)q for the 4 int8 codes of x. Each code
 // q becomes the half 1024 + (q + 128) (exponent 0x64 over the byte q ^ 0x80, built with
@@ -249,61 +222,20 @@ __device__ __forceinline__ void op_q8x4(uint32_t x, _Float16 s, _Float16* o) {
   o[3] = pb[1];
 }
 
-template <int FMT>
-__device__ __forceinline__ void op_store_w(const WRaw<FMT>& r, _Float16* Bs, int tid) {
-  _Float16* dst = Bs + (tid >> 1) * OP_LDK + 32 * (tid & 1);
-  if constexpr (FMT == 2) {
-    const _Float16 s = (_Float16)h2f(r.sm & 0xffff), m = (_Float16)h2f(r.sm >> 16);
-    const uint32_t x[4] = {r.b[0].x, r.b[0].y, r.b[0].z, r.b[0].w};
-    _Float16 o[32];
+// q4 dequantization, the 8 weights of a dword: s * q + m. Nibble pairs under the exponent
+// byte 0x64 are the halves 1024 + q; 1024 off is exact, then one fused f16 multiply-add.
+__device__ __forceinline__ void op_q4x8(uint32_t x, _Float16 s, _Float16 m, _Float16* o) {
+  const op_h2 k = {(_Float16)1024.f, (_Float16)1024.f}, sc = {s, s}, mn = {m, m};
 #pragma unroll
-    for (int i = 0; i < 16; i++) {
-      const uint32_t byte = (x[i >> 2] >> (8 * (i & 3))) & 0xff;
-      o[2 * i] = s * (_Float16)(float)(byte & 15) + m;
-      o[2 * i + 1] = s * (_Float16)(float)(byte >> 4) + m;
-    }
-#pragma unroll
-    for (int i = 0; i < 4; i++) *(uint4*)(dst + 8 * i) = *(const uint4*)(o + 8 * i);
-  } else if constexpr (FMT == 1) {
-    const _Float16 s = (_Float16)h2f(r.sm);
-    const uint32_t x[8] = {r.b[0].x, r.b[0].y, r.b[0].z, r.b[0].w, r.b[1].x, r.b[1].y, r.b[1].z, r.b[1].w};
-    _Float16 o[32];
-#pragma unroll
-    for (int i = 0; i < 8; i++) op_q8x4(x[i], s, o + 4 * i);
-#pragma unroll
-    for (int i = 0; i < 4; i++) *(uint4*)(dst + 8 * i) = *(const uint4*)(o + 8 * i);
-  } else {
-#pragma unroll
-    for (int i = 0; i < 4; i++) *(uint4*)(dst + 8 * i) = r.b[i];
+  for (int i = 0; i < 4; i++) {
+    const op_h2 q = __builtin_bit_cast(op_h2, ((x >> (4 * i)) & 0x000f000fu) | 0x64006400u) - k;
+    const op_h2 v = __builtin_elementwise_fma(q, sc, mn);
+    o[2 * i] = v[0];
+    o[2 * i + 1] = v[1];
   }
 }
 
-// A tile: BM rows x 64 halves; thread i (< BM * 8) carries 16 bytes (rows >= M read row
-// M - 1: finite, and their outputs are unused). Every thread loads (the surplus ones a
-// duplicate), so that the number of loads in flight never depends on a branch.
-template <int BM>
-struct ARaw {
-  uint4 v[(BM * 8 + 255) / 256];
-};
-template <int BM>
-__device__ __forceinline__ void op_fetch_a(const __half* A, int M, int K, int m0, int k0, int tid, ARaw<BM>& r) {
-#pragma unroll
-  for (int u = 0; u < (BM * 8 + 255) / 256; u++) {
-    const int i = (tid + 256 * u) & (BM * 8 - 1);
-    const int row = min(m0 + (i >> 3), M - 1);
-    r.v[u] = gld((const uint4*)(A + (size_t)row * K + k0) + (i & 7));
-  }
-}
-template <int BM>
-__device__ __forceinline__ void op_store_a(const ARaw<BM>& r, _Float16* As, int tid) {
-#pragma unroll
-  for (int u = 0; u < (BM * 8 + 255) / 256; u++) {
-    const int i = tid + 256 * u;
-    if (i < BM * 8) *(uint4*)(As + (i >> 3) * OP_LDK + 8 * (i & 7)) = r.v[u];
-  }
-}
-
-// ---- epilogues (shared by the fused GEMM and the split-K reduction) ---------------------
+// ---- epilogues ---------------------
 // QKV: one rotary block b = columns 32 b .. +31 holds dims d (x0, columns 32 b + i) and
 // d + 32 (x1, columns 32 b + 16 + i) of head b / 2 (Convert.swift:236-244); q heads 0-13,
 // k 14-15, v 16-17: bias, RoPE at the row's position, then q or the K / V cache slot.
@@ -437,17 +369,6 @@ __device__ __forceinline__ void op_gemm_epilogue(const OpGemmArgs& a, const OpHd
   }
 }
 
-// Workgroup: 256 threads = 4 waves; a wave owns 32 columns (two 16-column MFMA tiles) of
-// the 128-column tile and all BM rows. blockIdx.z selects a K slice of `ksteps` 64-column
-// steps; with more than one slice the kernel writes fp32 partials [slice][M][N] and
-// op_epi_kernel reduces them in slice order and applies the epilogue.
-// DEPTH > 1: the operands of the next DEPTH k-steps are in flight (a register ring) while
-// the current one is multiplied, and the LDS tiles are double-buffered, so one barrier per
-// k-step orders both their reuse and their filling; it waits for LDS traffic only (a full
-// __syncthreads would also drain the ring's loads). DEPTH 1: one k-step ahead, one LDS
-// buffer, two barriers per k-step, half the LDS and fewer registers: more workgroups per
-// CU, which is what the many-tile prefill gate/up GEMM needs (25.6 vs 40.7 us at 512 rows,
-// f16), while the ring wins where the tiles are few (O and down: 14.6 vs 17.0 us).
 // Tile of a prefill GEMM workgroup (grid: column tiles x row tiles x K slices). Workgroups
 // are dealt to the 8 XCDs round-robin (workgroup id mod 8), and each XCD has its own L2, so
 // the tiles are renumbered: the order (K slice, column tile, row tile) is cut into 8
@@ -466,112 +387,6 @@ __device__ __forceinline__ OpTile op_tile_xcd() {
   const int u = c * (T >> 3) + min(c, T & 7) + k;   // XCD c holds ceil((T - c) / 8) workgroups
   const int y = u % ny, sl = u / ny;
   return {sl % nx, y, sl / nx};
-}
-
-template <int FMT, int BM, int EPI, int DEPTH, int NB = (DEPTH > 1 ? 2 : 1)>
-__global__ __launch_bounds__(256) void op_gemm_kernel(OpGemmArgs a) {
-  const OpHdr hd = op_hdr(a.c);
-  __shared__ __attribute__((aligned(16))) _Float16 As[NB][BM * OP_LDK];
-  __shared__ __attribute__((aligned(16))) _Float16 Bs[NB][OP_BN * OP_LDK];
-  __shared__ uint64_t red[4][16];
-  constexpr int TM = BM / 16;
-  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-  const int kg = lane >> 4, n = lane & 15;
-  // (the gate/up GEMM keeps the dispatch order: renumbered it ran 1.5-10% slower, measured)
-  const OpTile tl = BM == 64 && EPI != OP_SILU ? op_tile_xcd() : OpTile{(int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z};
-  const int n0 = tl.x * OP_BN, m0 = tl.y * BM;
-  const int K = a.W.K;
-  const int kb = tl.z * a.ksteps * OP_BK, ke = min(K, kb + a.ksteps * OP_BK);
-  const int ns = (ke - kb) / OP_BK;
-  v4f acc[TM][2];
-#pragma unroll
-  for (int i = 0; i < TM; i++) {
-    acc[i][0] = (v4f){0.f, 0.f, 0.f, 0.f};
-    acc[i][1] = (v4f){0.f, 0.f, 0.f, 0.f};
-  }
-  if constexpr (DEPTH == 1) {
-    WRaw<FMT> wr;
-    ARaw<BM> ar;
-    op_fetch_w<FMT>(a.W, n0, kb, tid, wr);
-    op_fetch_a<BM>(a.A, a.M, K, m0, kb, tid, ar);
-    for (int k0 = kb; k0 < ke; k0 += OP_BK) {
-      op_store_a<BM>(ar, As[0], tid);
-      op_store_w<FMT>(wr, Bs[0], tid);
-      __syncthreads();
-      if (k0 + OP_BK < ke) {
-        op_fetch_w<FMT>(a.W, n0, k0 + OP_BK, tid, wr);
-        op_fetch_a<BM>(a.A, a.M, K, m0, k0 + OP_BK, tid, ar);
-      }
-#pragma unroll
-      for (int ks = 0; ks < 2; ks++) {
-        v8h bf[2];
-#pragma unroll
-        for (int j = 0; j < 2; j++) bf[j] = *(const v8h*)(Bs[0] + (32 * w + 16 * j + n) * OP_LDK + 32 * ks + 8 * kg);
-#pragma unroll
-        for (int i = 0; i < TM; i++) {
-          const v8h af = *(const v8h*)(As[0] + (16 * i + n) * OP_LDK + 32 * ks + 8 * kg);
-#pragma unroll
-          for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af, bf[j], acc[i][j], 0, 0, 0);
-        }
-      }
-      __syncthreads();
-    }
-    op_gemm_epilogue<BM, EPI>(a, hd, acc, m0, n0, tl.z, w, kg, n, red);
-    return;
-  }
-  constexpr int OP_DEPTH = DEPTH;
-  // Ring loads are unconditional (steps past the slice reload its last one), so that the
-  // compiler can count the loads in flight and wait for the oldest slot only.
-  WRaw<FMT> wr[OP_DEPTH];
-  ARaw<BM> ar[OP_DEPTH];
-#pragma unroll
-  for (int d = 0; d < OP_DEPTH; d++) {
-    const int k0 = kb + min(d, ns - 1) * OP_BK;
-    op_fetch_w<FMT>(a.W, n0, k0, tid, wr[d]);
-    op_fetch_a<BM>(a.A, a.M, K, m0, k0, tid, ar[d]);
-    __builtin_amdgcn_sched_barrier(0);   // issue order = slot order (the waits count on it)
-  }
-  // One k-step from ring slot d (st: the step's index in the slice); `refetch` refills the
-  // slot with step st + OP_DEPTH (clamped: the last round reloads the slice's last step).
-  auto kstep = [&](int d, int st, bool refetch) {
-    _Float16* as = As[(d & 1) % NB];
-    _Float16* bs = Bs[(d & 1) % NB];
-    if constexpr (NB == 1) lds_barrier();   // one buffer: every wave is done with the last step
-    op_store_a<BM>(ar[d], as, tid);
-    op_store_w<FMT>(wr[d], bs, tid);
-    lds_barrier();   // LDS only: the ring's HBM loads stay in flight
-    if (refetch) {
-      const int k0 = kb + min(st + OP_DEPTH, ns - 1) * OP_BK;
-      __builtin_amdgcn_sched_barrier(0);
-      op_fetch_w<FMT>(a.W, n0, k0, tid, wr[d]);
-      op_fetch_a<BM>(a.A, a.M, K, m0, k0, tid, ar[d]);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-#pragma unroll
-    for (int ks = 0; ks < 2; ks++) {
-      v8h bf[2];
-#pragma unroll
-      for (int j = 0; j < 2; j++) bf[j] = *(const v8h*)(bs + (32 * w + 16 * j + n) * OP_LDK + 32 * ks + 8 * kg);
-#pragma unroll
-      for (int i = 0; i < TM; i++) {
-        const v8h af = *(const v8h*)(as + (16 * i + n) * OP_LDK + 32 * ks + 8 * kg);
-#pragma unroll
-        for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af, bf[j], acc[i][j], 0, 0, 0);
-      }
-    }
-  };
-  // Whole rounds of OP_DEPTH steps with no branch between their loads (so every path into
-  // the loop head has the same loads in flight and the waits stay partial), then the tail
-  // from the ring without refills.
-  int s0 = 0;
-  for (; s0 + OP_DEPTH <= ns; s0 += OP_DEPTH) {
-#pragma unroll
-    for (int d = 0; d < OP_DEPTH; d++) kstep(d, s0 + d, true);
-  }
-#pragma unroll
-  for (int d = 0; d < OP_DEPTH - 1; d++)
-    if (s0 + d < ns) kstep(d, s0 + d, false);
-  op_gemm_epilogue<BM, EPI>(a, hd, acc, m0, n0, tl.z, w, kg, n, red);
 }
 
 // ---- prefill GEMM, q8 / f16: operands streamed from memory into an LDS ring --------------
@@ -618,11 +433,11 @@ __device__ __forceinline__ void op_lds_dma4(const void* g, const void* lds) {
 template <int FMT, int BM>
 struct OpRing {                                  // sizes in 16-byte units
   static constexpr int A = BM * 8;
-  static constexpr int B = FMT == 0 ? 1024 : 512;
-  static constexpr int SC = FMT == 1 ? 32 : 0;
+  static constexpr int B = FMT == 0 ? 1024 : (FMT == 1 ? 512 : 256);
+  static constexpr int SC = FMT == 0 ? 0 : 32;
   static constexpr int N = A + B + SC;
   static constexpr int LA = A >= 256 ? A / 256 : 1;   // A loads per thread (BM 16: waves 2, 3 repeat 0, 1)
-  static constexpr int L = LA + B / 256 + (FMT == 1 ? 1 : 0);   // loads per thread and stage
+  static constexpr int L = LA + B / 256 + (FMT == 0 ? 0 : 1);   // loads per thread and stage
 };
 
 // Thread tid's loads of the k-step at k0 into stage st (rows >= M read row M - 1).
@@ -638,13 +453,13 @@ __device__ __forceinline__ void op_ring_load(const OpGemmArgs& a, int m0, int n0
     const int row = min(m0 + ((p >> 7) << 4) + (p & 15), a.M - 1);
     op_lds_dma16(a.A + (size_t)row * K + k0 + 8 * ((p >> 4) & 7), st + ((256 * u + wb) & (R::A - 1)));
   }
-  const uint4* blk = (const uint4*)(a.W.w + op_wt_off(n0, k0, K, FMT == 0 ? 2 : 1));
+  const uint4* blk = (const uint4*)(a.W.w + (FMT == 2 ? op_w4_off(n0, k0, K) : op_wt_off(n0, k0, K, FMT == 0 ? 2 : 1)));
 #pragma unroll
   for (int u = 0; u < R::B / 256; u++)
     op_lds_dma16(blk + 256 * u + tid, st + R::A + 256 * u + wb);
-  if constexpr (FMT == 1) {   // 64 dwords per wave: all of them (qg 64), or half (qg 32: waves 0, 2 the first)
-    const int off = a.W.qg == 32 ? ((tid >> 6) & 1) * 64 : 0;
-    const uint32_t* sc = (const uint32_t*)(a.W.s + op_st_off(n0, k0, K, a.W.qg));
+  if constexpr (FMT != 0) {   // 64 dwords per wave: all of them (q8, qg 64), or half (q4; q8, qg 32: waves 0, 2 the first)
+    const int off = FMT == 2 || a.W.qg == 32 ? ((tid >> 6) & 1) * 64 : 0;
+    const uint32_t* sc = FMT == 2 ? (const uint32_t*)a.W.s + op_st_off(n0, k0, K, 64) : (const uint32_t*)(a.W.s + op_st_off(n0, k0, K, a.W.qg));
     op_lds_dma4(sc + off + (tid & 63), (uint32_t*)(st + R::A + R::B) + off);
   }
 }
@@ -661,6 +476,13 @@ __device__ __forceinline__ void op_ring_mma(const uint4* st, int w, int kg, int 
       const int c16 = 2 * w + j;   // 16-row sub-tile of the weight block
       if constexpr (FMT == 0) {
         bf[j] = u4_to_v8h(st[R::A + c16 * 128 + ((kg & 1) * 4 + 2 * ks + (kg >> 1)) * 16 + n]);
+      } else if constexpr (FMT == 2) {
+        const uint32_t x = ((const uint32_t*)(st + R::A + c16 * 32))[((2 * ks + (kg >> 1)) * 16 + n) * 2 + (kg & 1)];
+        const uint32_t sm = ((const uint32_t*)(st + R::A + R::B))[16 * c16 + n];
+        _Float16 o[8];
+        op_q4x8(x, (_Float16)h2f(sm & 0xffff), (_Float16)h2f(sm >> 16), o);
+#pragma unroll
+        for (int i = 0; i < 8; i++) bf[j][i] = o[i];
       } else {
         const uint2 q = ((const uint2*)(st + R::A + c16 * 64 + (2 * ks + (kg >> 1)) * 16 + n))[kg & 1];
         const uint16_t* sc = (const uint16_t*)(st + R::A + R::B);
@@ -705,7 +527,7 @@ __device__ __forceinline__ void op_ring_wait(int later) {
 // the 128-column tile and all BM rows).
 template <int FMT, int BM, int EPI, int ST>
 __global__ __launch_bounds__(256) void op_gemm_ring_kernel(OpGemmArgs a) {
-  static_assert(FMT != 2 && ST >= 2 && ST <= 8 && BM >= 16 && BM <= 64 && (EPI != OP_LMH || BM == 16), "ring GEMM shape");
+  static_assert(ST >= 2 && ST <= 8 && BM >= 16 && BM <= 64 && (EPI != OP_LMH || BM == 16), "ring GEMM shape");
   using R = OpRing<FMT, BM>;
   const OpHdr hd = op_hdr(a.c);
 #define OP_RING_ARR(i) __shared__ __attribute__((aligned(16))) uint4 r##i[ST > i ? R::N : 1];
@@ -770,227 +592,6 @@ __global__ __launch_bounds__(256) void op_gemm_ring_kernel(OpGemmArgs a) {
   else op_gemm_epilogue<BM, EPI>(a, hd, acc, m0, n0, tl.z, w, kg, n, red);
 }
 
-// ---- GEMM of passes of up to 16 rows --------------------------------------------------
-// Workgroup: 4 waves, wave w owns columns n0 + 32 w .. + 31 (two 16-column MFMA tiles) and
-// rows 0-15. The A rows of the K slice sit in LDS for the whole kernel (filled once, one
-// barrier); each wave loads its own weight operands straight into registers (no LDS, no
-// barrier in the k loop), OP_SDEPTH(FMT) k-steps of them in flight. Within a k-step lane (kg, n)
-// takes columns 16 kg .. 16 kg + 15 of the 64 (8 for each of the two MFMAs), a permutation
-// of k applied to A and W alike. With SILU the A operand is the SwiGLU unit
-// f16(silu(g) * u) of the gate/up GEMM's K-slice partials (summed in slice order, as
-// op_epi_kernel does), so that no separate SiLU kernel runs. The host uses it for that
-// down projection only: for the other small-pass GEMMs the LDS-tiled op_gemm_kernel<.., 16,
-// ..> measured as fast (q8) or faster (f16: about 3 us per step-kernel).
-#define OP_SDEPTH(FMT) ((FMT) == 0 ? 4 : 8)   // f16 k-steps carry twice the bytes of q8 ones
-#define OP_SMAXK 1024   // K slice columns at most (16 k-steps)
-
-template <int FMT>
-struct BOp {   // one k-step's weights of one lane for the wave's two column tiles
-  uint4 q[2][FMT == 0 ? 2 : 1];   // q4: .x .y hold the 16 nibbles
-  // q8: scale (kept 16-bit: widening the loaded value would wait for it at once);
-  // q4: (scale, min)
-  std::conditional_t<FMT == 2, uint32_t, uint16_t> s[2];
-};
-template <int FMT>
-__device__ __forceinline__ void op_fetch_b(const OpMat& W, int col0, int k0, int kg, int n, BOp<FMT>& b) {
-#pragma unroll
-  for (int j = 0; j < 2; j++) {
-    const size_t row = (size_t)(col0 + 16 * j + n);
-    const int k = k0 + 16 * kg;
-    if constexpr (FMT == 2) {
-      const uint2 v = gld((const uint2*)(W.w + row * (W.K / 2) + k / 2));
-      b.q[j][0] = make_uint4(v.x, v.y, 0u, 0u);
-      b.s[j] = gld((const uint32_t*)(W.s + (row * (W.K / 64) + k / 64) * 2));
-    } else if constexpr (FMT == 1) {
-      b.q[j][0] = gld((const uint4*)(W.w + op_wt_off((int)row, k, W.K, 1)));
-      b.s[j] = gld(W.s + op_st_off((int)row, k, W.K, W.qg));
-    } else {
-      b.q[j][0] = gld((const uint4*)(W.w + op_wt_off((int)row, k, W.K, 2)));
-      b.q[j][1] = gld((const uint4*)(W.w + op_wt_off((int)row, k + 8, W.K, 2)));
-    }
-  }
-}
-// the 8 f16 operand values of MFMA half ks (k = 16 kg + 8 ks ..) of column tile j
-template <int FMT>
-__device__ __forceinline__ v8h op_bvals(const BOp<FMT>& b, int j, int ks) {
-  v8h o;
-  if constexpr (FMT == 2) {
-    const _Float16 sc = (_Float16)h2f(b.s[j] & 0xffff), mn = (_Float16)h2f(b.s[j] >> 16);
-    const uint32_t x = ks == 0 ? b.q[j][0].x : b.q[j][0].y;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const uint32_t byte = (x >> (8 * i)) & 0xff;
-      o[2 * i] = sc * (_Float16)(float)(byte & 15) + mn;
-      o[2 * i + 1] = sc * (_Float16)(float)(byte >> 4) + mn;
-    }
-  } else if constexpr (FMT == 1) {
-    const _Float16 sc = (_Float16)h2f(b.s[j]);
-    const uint32_t x0 = ks == 0 ? b.q[j][0].x : b.q[j][0].z, x1 = ks == 0 ? b.q[j][0].y : b.q[j][0].w;
-    _Float16 h[8];
-    op_q8x4(x0, sc, h);
-    op_q8x4(x1, sc, h + 4);
-#pragma unroll
-    for (int i = 0; i < 8; i++) o[i] = h[i];
-  } else {
-    o = u4_to_v8h(b.q[j][ks]);
-  }
-  return o;
-}
-
-template <int FMT, int EPI, bool SILU, int NWV = 4>
-__global__ __launch_bounds__(64 * NWV) void op_gemv_kernel(OpGemmArgs a) {
-  // NWV 4: four waves, 32 columns each. NWV 2 (the unsplit QKV GEMM): two waves share 32
-  // columns and split the K steps in halves, added (wave 0's + wave 1's) before the
-  // epilogue, which wave 0 applies.
-  static_assert(NWV == 4 || (NWV == 2 && EPI == OP_QKV), "two-wave workgroups: the unsplit QKV GEMM");
-  constexpr bool KS2 = NWV == 2;
-  constexpr int NT = 64 * NWV;
-  const OpHdr hd = op_hdr(a.c);
-  __shared__ __attribute__((aligned(16))) _Float16 As[16 * (OP_SMAXK + 8)];
-  __shared__ uint64_t red[4][16];
-  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-  const int kg = lane >> 4, n = lane & 15;
-  const int n0 = blockIdx.x * (KS2 ? 32 : 32 * NWV), col0 = n0 + (KS2 ? 0 : 32 * w);
-  // QKV: the rotary rows of this lane's rows 4 kg + r at the expected position (pos_hint + row)
-  float2 cs[4];
-  if constexpr (EPI == OP_QKV) {
-#pragma unroll
-    for (int r = 0; r < 4; r++)
-      cs[r] = gld(a.c.rope + (size_t)min(a.pos_hint + 4 * kg + r, a.c.maxctx - 1) * 32 + ((col0 >> 5) & 1) * 16 + n);
-  }
-  const int K = a.W.K;
-  const int kb = blockIdx.z * a.ksteps * OP_BK, ke = min(K, kb + a.ksteps * OP_BK);
-  const int nsa = (ke - kb) / OP_BK, kw = ke - kb;
-  const int lda = kw + 8;   // LDS row stride (halves)
-  // this wave's k-steps: all of the slice, or (KS2) its half
-  const int s_lo = KS2 ? w * nsa / NWV : 0;
-  const int ns = KS2 ? (w + 1) * nsa / NWV - s_lo : nsa;
-  const int kbw = kb + s_lo * OP_BK;   // the wave's first column
-  constexpr int SD = OP_SDEPTH(FMT);
-  BOp<FMT> ring[SD];
-#pragma unroll
-  for (int d = 0; d < SD; d++) {
-    op_fetch_b<FMT>(a.W, col0, kbw + min(d, ns - 1) * OP_BK, kg, n, ring[d]);
-    __builtin_amdgcn_sched_barrier(0);   // issue order = slot order (the waits count on it)
-  }
-  // A rows 0 .. M-1 of the slice into LDS (rows >= M are left as they are: their outputs
-  // are never stored)
-  if constexpr (!SILU) {
-    const int per = kw / 8;   // uint4 per row
-    for (int i = tid; i < a.M * per; i += NT) {
-      const int m = i / per, c8 = i - m * per;
-      *(uint4*)(As + m * lda + 8 * c8) = gld((const uint4*)(a.A + (size_t)m * K + kb) + c8);
-    }
-  } else {
-    // units kb + 2 p, kb + 2 p + 1 of row m: gate/up columns 2 kb + 4 p .. + 3 (g, g, u, u)
-    const int per = kw / 2, N2 = 2 * K;
-    for (int i = tid; i < a.M * per; i += NT) {
-      const int m = i / per, p = i - m * per;
-      float4 pz[OP_MAXS];
-#pragma unroll
-      for (int z = 0; z < OP_MAXS; z++)
-        if (z < a.aS) pz[z] = gld((const float4*)(a.apart + ((size_t)z * a.M + m) * N2 + 2 * kb) + p);
-      float4 v = pz[0];
-#pragma unroll
-      for (int z = 1; z < OP_MAXS; z++)
-        if (z < a.aS) {
-          v.x += pz[z].x;
-          v.y += pz[z].y;
-          v.z += pz[z].z;
-          v.w += pz[z].w;
-        }
-      As[m * lda + 2 * p] = (_Float16)__float2half(v.x / (1.0f + expf(-v.x)) * v.z);
-      As[m * lda + 2 * p + 1] = (_Float16)__float2half(v.y / (1.0f + expf(-v.y)) * v.w);
-    }
-  }
-  __syncthreads();
-  v4f acc[1][2];
-  acc[0][0] = (v4f){0.f, 0.f, 0.f, 0.f};
-  acc[0][1] = (v4f){0.f, 0.f, 0.f, 0.f};
-  auto kstep = [&](int d, int st, bool refetch) {
-    v8h bf[2][2];
-#pragma unroll
-    for (int j = 0; j < 2; j++)
-#pragma unroll
-      for (int ks = 0; ks < 2; ks++) bf[j][ks] = op_bvals<FMT>(ring[d], j, ks);
-    if (refetch) {
-      __builtin_amdgcn_sched_barrier(0);
-      op_fetch_b<FMT>(a.W, col0, kbw + min(st + SD, ns - 1) * OP_BK, kg, n, ring[d]);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-#pragma unroll
-    for (int ks = 0; ks < 2; ks++) {
-      const v8h af = *(const v8h*)(As + n * lda + (s_lo + st) * OP_BK + 16 * kg + 8 * ks);
-#pragma unroll
-      for (int j = 0; j < 2; j++) acc[0][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af, bf[j][ks], acc[0][j], 0, 0, 0);
-    }
-  };
-  int s0 = 0;
-  for (; s0 + SD <= ns; s0 += SD) {
-#pragma unroll
-    for (int d = 0; d < SD; d++) kstep(d, s0 + d, true);
-  }
-#pragma unroll
-  for (int d = 0; d < SD - 1; d++)
-    if (s0 + d < ns) kstep(d, s0 + d, false);
-  if constexpr (KS2) {
-    __shared__ v4f kacc[NWV][2][64];
-    if (w > 0) {
-      kacc[w][0][lane] = acc[0][0];
-      kacc[w][1][lane] = acc[0][1];
-    }
-    __syncthreads();
-    if (w > 0) return;
-#pragma unroll
-    for (int ww = 1; ww < NWV; ww++)
-#pragma unroll
-      for (int jj = 0; jj < 2; jj++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) acc[0][jj][r] = acc[0][jj][r] + kacc[ww][jj][lane][r];
-    op_gemm_epilogue<16, EPI>(a, hd, acc, 0, n0, (int)blockIdx.z, 0, kg, n, red, a.pos_hint, cs);
-  } else {
-    op_gemm_epilogue<16, EPI>(a, hd, acc, 0, n0, (int)blockIdx.z, w, kg, n, red, a.pos_hint, cs);
-  }
-}
-
-// Split-K reduction: sum of the slices' partials in slice order, then the epilogue.
-// RESID / SILU / QKV: one thread per output column / unit / rotary pair of a row.
-template <int EPI>
-__global__ __launch_bounds__(256) void op_epi_kernel(OpGemmArgs a, int S) {
-  const OpHdr hd = op_hdr(a.c);
-  const int N = a.W.N;
-  const int per = EPI == OP_RESID ? N : N / 2;   // SILU: units; QKV: pairs
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= a.M * per) return;
-  const int m = i / per, j = i % per;
-  // every slice's partial in flight at once, then added in slice order
-  auto sum = [&](int col) {
-    float pz[OP_MAXS];
-#pragma unroll
-    for (int z = 0; z < OP_MAXS; z++) pz[z] = z < S ? gld(a.part + ((size_t)z * a.M + m) * N + col) : 0.f;
-    float v = pz[0];
-#pragma unroll
-    for (int z = 1; z < OP_MAXS; z++)
-      if (z < S) v += pz[z];
-    return v;
-  };
-  if constexpr (EPI == OP_RESID) {
-    float* r = a.resid + (size_t)m * ILL_H + j;
-    const float x = gld(r), y = sum(j);
-    if (!hd.done) gst(r, x + y);
-  } else if constexpr (EPI == OP_SILU) {
-    const int q = j >> 1, r = j & 1;
-    const float g = sum(4 * q + r), u = sum(4 * q + 2 + r);
-    if (!hd.done) epi_silu(a.c, m, j, g, u);
-  } else if constexpr (EPI == OP_QKV) {
-    const int b = j >> 4, ii = j & 15;
-    const int at = min(a.pos_hint + m, a.c.maxctx - 1);   // a chain row's expected position
-    const float2 cs = gld(a.c.rope + (size_t)at * 32 + (b & 1) * 16 + ii);
-    const float x0 = sum(32 * b + ii), x1 = sum(32 * b + 16 + ii);
-    if (!hd.done) epi_qkv(a.c, hd, a.layer, m, b, ii, x0, x1, at, cs);
-  }
-}
-
 // Residual split-K reduction fused with the RMSNorm that reads the updated residual, for
 // passes of up to 16 rows: one workgroup per row m, one thread per column. x[m] += the
 // slices' partials (added in slice order, as op_epi_kernel); then, for rows m >= row0,
@@ -1024,24 +625,6 @@ __global__ __launch_bounds__(ILL_H) void op_epi_norm_kernel(OpGemmArgs a, int S,
   gst((uint16_t*)(a.c.xn + (size_t)(m - row0) * ILL_H + j), (uint16_t)__half_as_ushort(__float2half(v * scale * g)));
 }
 
-// ---- attention of passes of up to 16 rows -------------------------------------------------
-// Row t attends to virtual positions 0 .. L-1, L = pos + depth(t) + 1; position p lives in
-// cache slot p below pos and in slot pos + (the row on t's path at depth p - pos) above
-// (tree passes; chains use slot p). The row's 64-position chunks are dealt to 64 slots:
-// chunk c to slot (split s = (c / 16) % 8, wave w = c % 8), so a context of up to 1024
-// positions is all split 0. Slot (s, w) folds its chunks in increasing order with the pass
-// kernel's rule, the eight slots of split s are combined against their maximum (in w
-// order), then the eight splits against theirs (in s order).
-// The grouping depends only on the row's L, not on M or on how the work is launched, so a
-// row decoded alone and the same row inside a 16-row pass give identical bits.
-// One workgroup of 8 waves per (row t, query head h, part j < nsplit) runs the splits j,
-// j + nsplit, ...: with nsplit = 1 it finishes the row; otherwise it stores its split
-// states and op_attn_combine_kernel finishes the row. (The host picks nsplit from the
-// context length it expects; any value gives the same result.)
-#define OP_NSPLIT 8
-#define OP_SPLIT_W 66   // scratch words per split state: m, l, o[64]
-#define OP_VST 72       // LDS stride (halves) of a staged V row
-
 // (m, l, o) of n states combined against their maximum, in index order; states with
 // m = -inf (no positions) add nothing, and if all are empty the result is empty too.
 template <int N>
@@ -1063,322 +646,6 @@ __device__ __forceinline__ void att_combine(const float* m, const float* l, cons
   oo = acc;
 }
 
-// The O projection of one (row, head) folded into the attention kernel (passes of up to 16
-// rows, one attention split): wave w computes output columns 112 w + lane and
-// 112 w + 64 + lane (lane < 48) of W_o[:, 64 h .. 64 h + 63] . ao, where ao is the head's
-// f16 output (LDS). Weights are dequantized as op_gemm_kernel does (q8: f16 s * q; f16 as
-// stored) and the 64 products are added in k order in fp32: the partial of slice h, which
-// op_epi_norm_kernel sums over the 14 heads in head order.
-template <int FMT>
-struct ORows {
-  uint4 q[2][FMT == 0 ? 8 : 4];
-  uint32_t s[2];   // q8: the scales of k 0-31 (low half) and 32-63 (high; equal for group 64)
-};
-// Woh: the head-major copy (OpLayerW::oh), so each load reads 1 KB contiguous over the lanes
-template <int FMT>
-__device__ __forceinline__ void orows_fetch(const OpMat& Woh, int h, int w, int lane, ORows<FMT>& o) {
-  constexpr int NC = FMT == 0 ? 8 : 4;   // 16-byte chunks of a row's 64 columns
-#pragma unroll
-  for (int u = 0; u < 2; u++) {
-    const int r = min(112 * w + 64 * u + lane, ILL_H - 1);
-    const uint4* src = (const uint4*)Woh.w + (size_t)h * NC * ILL_H + r;
-#pragma unroll
-    for (int i = 0; i < NC; i++) o.q[u][i] = gld(src + (size_t)i * ILL_H);
-    if constexpr (FMT == 1) o.s[u] = gld((const uint32_t*)Woh.s + (size_t)h * ILL_H + r);
-  }
-}
-template <int FMT>
-__device__ __forceinline__ void orows_apply(const ORows<FMT>& o, const _Float16* ao, int w, int lane, float* dst) {
-#pragma unroll
-  for (int u = 0; u < 2; u++) {
-    const int r = 112 * w + 64 * u + lane;
-    float acc = 0.f;
-#pragma unroll
-    for (int i = 0; i < (FMT == 0 ? 8 : 4); i++) {
-      const uint32_t x[4] = {o.q[u][i].x, o.q[u][i].y, o.q[u][i].z, o.q[u][i].w};
-      constexpr int PER = FMT == 0 ? 8 : 16;   // k values per uint4
-      _Float16 wq[FMT == 1 ? 16 : 1];
-      if constexpr (FMT == 1) {   // k = 16 i + e: the scale of k / 32 = i / 2
-        const _Float16 sc = (_Float16)h2f((uint16_t)(o.s[u] >> (16 * (i >> 1))));
-#pragma unroll
-        for (int q = 0; q < 4; q++) op_q8x4(x[q], sc, wq + 4 * q);
-      }
-#pragma unroll
-      for (int e = 0; e < PER; e++) {
-        const int k = PER * i + e;
-        _Float16 wv;
-        if constexpr (FMT == 1) wv = wq[e];
-        else wv = __ushort_as_half((unsigned short)((x[e >> 1] >> (16 * (e & 1))) & 0xffff));
-        acc = fmaf((float)wv, (float)ao[k], acc);
-      }
-    }
-    if (u == 0 || lane < 48) dst[r] = acc;
-  }
-}
-
-template <int FMT>
-__global__ __launch_bounds__(64 * ILL_WAVES) void op_attn_kernel(OpCtx c, int layer, int M, int nsplit, float* scratch,
-                                                               OpMat Wo, float* opart) {
-  __shared__ __attribute__((aligned(16))) float qs[ILL_WAVES][64];   // a copy per wave
-  __shared__ __attribute__((aligned(16))) float ps[ILL_WAVES][64];
-  __shared__ int path[16];
-  __shared__ float cm[OP_NSPLIT][ILL_WAVES], cl[OP_NSPLIT][ILL_WAVES], co[OP_NSPLIT][ILL_WAVES][64];
-  __shared__ float sm[OP_NSPLIT], sl[OP_NSPLIT], so[OP_NSPLIT][64];
-  __shared__ __attribute__((aligned(16))) uint16_t vstage[ILL_WAVES][64 * OP_VST];   // tree passes: V rows
-  __shared__ _Float16 aoh[64];   // with opart: the head's output, the O projection's input
-  const OpHdr hd = op_hdr(c);
-  constexpr bool SWZ = FMT != 2;   // the cache layout of the q8 / f16 engines (ill_common.h)
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int rh = blockIdx.x / nsplit, j = blockIdx.x % nsplit;
-  const int t = rh / ILL_NH, h = rh % ILL_NH, g = h / 7;
-  const float qv = gld(c.q + (size_t)t * ILL_H + h * 64 + lane);   // before the K/V loads
-  // with opart (nsplit 1, q8 / f16) the O projection follows (this wave's W_o rows are
-  // fetched when the chunk loop is done: held from the start they would spill)
-  constexpr bool OFUSE = FMT != 2;
-  const bool fused = OFUSE && opart != nullptr;
-  ORows<OFUSE ? FMT : 1> orw;
-  const uint16_t* kb = c.kc + ((size_t)layer * ILL_NKV + g) * c.maxctx * 64;
-  const uint16_t* vb = c.vt + ((size_t)layer * ILL_NKV + g) * (c.maxctx / 64) * 4096;
-  // The wave's first chunk (split j, chunk 16 j + w) at its plain slots, issued before the
-  // header is waited for; it is used unless the chunk lies past the row's positions or
-  // holds pass rows of a tree pass (their slots come from the path table).
-  uint4 kv[8], vv[8];
-  const int ch0 = 16 * j + w;
-  {
-    const int ks = min(64 * ch0 + lane, c.maxctx - 1), vc = min(ch0, c.maxctx / 64 - 1);
-#pragma unroll
-    for (int i = 0; i < 8; i++) kv[i] = gld((const uint4*)(kb + kv_k_off(ks, 8 * i, SWZ)));
-#pragma unroll
-    for (int i = 0; i < 8; i++) vv[i] = gld((const uint4*)(vb + kv_v_off(64 * vc + 8 * i, lane, SWZ)));
-  }
-  const int pos = hd.pos;
-  const bool tree = hd.mode == ILL_MODE_TREE;
-  const int dep = op_depth(c, hd.mode, t);
-  const int L = pos + dep + 1;
-  const int nch = (L + 63) >> 6;
-  const int nne = min(OP_NSPLIT, (nch + 15) >> 4);   // splits 0 .. nne - 1 hold chunks
-  // chunk ch: the K row of position 64 ch + lane (slot remapped along the path in tree
-  // passes) and the V values of dim = lane
-  auto fetch = [&](int ch, uint4 (&kv)[8], uint4 (&vv)[8]) {
-    const int vp = 64 * ch + lane;
-    const int slot = min(vp < pos || !tree ? vp : pos + path[min(max(vp - pos, 0), 15)], c.maxctx - 1);
-#pragma unroll
-    for (int i = 0; i < 8; i++) kv[i] = gld((const uint4*)(kb + kv_k_off(slot, 8 * i, SWZ)));
-#pragma unroll
-    for (int i = 0; i < 8; i++) vv[i] = gld((const uint4*)(vb + kv_v_off(64 * ch + 8 * i, lane, SWZ)));
-  };
-  const bool early = j < nne && ch0 < nch && (!tree || 64 * ch0 + 63 < pos);
-  qs[w][lane] = qv * 0.125f;
-  if (w == 0 && lane < 16) {   // rows on t's path by depth (tree passes: depth <= 15)
-    int pr = lane;
-    if (tree) {
-      int r = t;
-      for (int d = dep; d >= 0; --d) {
-        if (d == lane) pr = r;
-        r = r > 0 ? gld(c.tree + ILL_TR_PARENT + r) : 0;
-      }
-    }
-    path[lane] = pr;
-  }
-  lds_barrier();   // path and qs visible; the chunk loads stay in flight
-#pragma unroll 1
-  for (int q = 0; q < OP_NSPLIT; q++) {
-    const int s = j + nsplit * q;
-    if (s >= nne) break;
-    float Mx = -INFINITY, Ls = 0.f, O = 0.f;
-    // this wave's chunks of split s: 128 r + 16 s + 8 b + w (r = 0, 1, ..., b = 0, 1) in
-    // order; the next one streams in while one is evaluated
-    auto chunk_of = [&](int i) { return 128 * (i >> 1) + 16 * s + 8 * (i & 1) + w; };
-    int ch = chunk_of(0);
-    if (ch < nch && !(q == 0 && early)) fetch(ch, kv, vv);
-    for (int ci = 0; ch < nch; ch = chunk_of(++ci)) {
-      uint4 kn[8], vn[8];
-      const int nx = chunk_of(ci + 1);
-      const bool more = nx < nch;
-      if (more) fetch(nx, kn, vn);
-      const int vp = 64 * ch + lane;
-      const bool valid = vp < L;
-      float sc = 0.f;
-      // q is re-read from LDS for every chunk (broadcast reads): held in registers it would
-      // push the two K/V buffers out of them
-      asm volatile("" ::: "memory");
-#pragma unroll
-      for (int i = 0; i < 8; i++) {
-        const uint32_t x[4] = {kv[i].x, kv[i].y, kv[i].z, kv[i].w};
-        const float4 qa = *(const float4*)&qs[w][8 * i], qb = *(const float4*)&qs[w][8 * i + 4];
-        const float qv[8] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w};
-#pragma unroll
-        for (int e = 0; e < 8; e++) sc = fmaf(qv[e], h2f(x[e >> 1] >> (16 * (e & 1))), sc);
-      }
-      sc = valid ? sc : -INFINITY;
-      const float mc = gmax<64>(sc);
-      const float p = valid ? att_exp(sc - mc) : 0.f;
-      const float lc = gsum<64>(p);
-      ps[w][lane] = p;
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      float oc = 0.f;
-      if (tree && 64 * ch + 63 >= pos) {   // wave-uniform: positions pos .. L-1 of the chunk
-        // take the V of the path rows' slots: this lane's V row goes through LDS, where
-        // those (at most 16) positions are replaced
-        uint16_t* vr = &vstage[w][lane * OP_VST];
-#pragma unroll
-        for (int i = 0; i < 8; i++) *(uint4*)(vr + 8 * i) = vv[i];
-        const int p0 = max(pos - 64 * ch, 0), p1 = min(L - 64 * ch, 64);
-        uint16_t pv[16];
-#pragma unroll
-        for (int k = 0; k < 16; k++) {
-          const int pp = p0 + k;
-          if (pp < p1) {
-            const int sl2 = pos + path[64 * ch + pp - pos];
-            pv[k] = gld(vb + kv_v_off(sl2, lane, SWZ));
-          }
-        }
-#pragma unroll
-        for (int k = 0; k < 16; k++)
-          if (p0 + k < p1) vr[p0 + k] = pv[k];
-#pragma unroll
-        for (int i = 0; i < 8; i++) vv[i] = *(const uint4*)(vr + 8 * i);
-      }
-#pragma unroll
-      for (int i = 0; i < 8; i++) {
-        const uint32_t x[4] = {vv[i].x, vv[i].y, vv[i].z, vv[i].w};
-#pragma unroll
-        for (int e = 0; e < 8; e++) {
-          const int pp = 8 * i + e, vq = 64 * ch + pp;
-          float v = h2f(x[e >> 1] >> (16 * (e & 1)));
-          v = vq < L ? v : 0.f;
-          oc = fmaf(ps[w][pp], v, oc);
-        }
-      }
-      __builtin_amdgcn_wave_barrier();
-      const AttScale k = att_scale(Mx, mc);
-      O = att_fold(O, oc, k);
-      Ls = att_fold(Ls, lc, k);
-      Mx = k.mn;
-      if (more) {
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-          kv[i] = kn[i];
-          vv[i] = vn[i];
-        }
-      }
-    }
-    if (lane == 0) {
-      cm[q][w] = Mx;
-      cl[q][w] = Ls;
-    }
-    co[q][w][lane] = O;
-  }
-  if constexpr (OFUSE)
-    if (fused) orows_fetch<FMT>(Wo, h, w, lane, orw);
-  __syncthreads();
-  // the head's output row: to c.ao, or (opart) through LDS into the O projection
-  auto emit = [&](float v) {
-    const __half hv = __float2half(v);
-    if (fused) aoh[lane] = (_Float16)hv;
-    else if (!hd.done) gst((uint16_t*)(c.ao + (size_t)t * ILL_H + h * 64 + lane), (uint16_t)__half_as_ushort(hv));
-  };
-  auto oproj = [&]() {
-    if constexpr (OFUSE) {
-      __syncthreads();
-      orows_apply<FMT>(orw, aoh, w, lane, opart + ((size_t)h * M + t) * ILL_H);
-    }
-  };
-  if (nsplit == 1 && nne == 1) {   // one split: its state is the row's (the general path
-    if (w == 0) {                  // below gives the same bits: scale 1, nothing added)
-      float o[ILL_WAVES];
-#pragma unroll
-      for (int ww = 0; ww < ILL_WAVES; ww++) o[ww] = co[0][ww][lane];
-      float mo, lo, oo;
-      att_combine<ILL_WAVES>(cm[0], cl[0], o, mo, lo, oo);
-      emit(oo / lo);
-    }
-    if (fused) oproj();
-    return;
-  }
-  // split states: wave q combines the slots of split j + nsplit q (empty splits: m = -inf)
-  const int nq = (OP_NSPLIT - j + nsplit - 1) / nsplit;
-  if (w < nq) {
-    if (j + nsplit * w >= nne) {   // no chunks: nothing was stored for it
-      if (lane == 0) {
-        cm[w][0] = -INFINITY;
-        cl[w][0] = 0.f;
-      }
-#pragma unroll
-      for (int ww = 1; ww < ILL_WAVES; ww++)
-        if (lane == 0) cm[w][ww] = -INFINITY;
-    }
-    float o[ILL_WAVES];
-#pragma unroll
-    for (int ww = 0; ww < ILL_WAVES; ww++) o[ww] = co[w][ww][lane];
-    float mo, lo, oo;
-    att_combine<ILL_WAVES>(cm[w], cl[w], o, mo, lo, oo);
-    if (nsplit == 1) {
-      if (lane == 0) {
-        sm[w] = mo;
-        sl[w] = lo;
-      }
-      so[w][lane] = oo;
-    } else {
-      float* dst = scratch + ((size_t)rh * OP_NSPLIT + j + nsplit * w) * OP_SPLIT_W;
-      if (lane == 0) {
-        dst[0] = mo;
-        dst[1] = lo;
-      }
-      dst[2 + lane] = oo;
-    }
-  }
-  if (nsplit > 1) return;
-  __syncthreads();
-  if (w == 0) {
-    float o[OP_NSPLIT];
-#pragma unroll
-    for (int q = 0; q < OP_NSPLIT; q++) o[q] = so[q][lane];
-    float mo, lo, oo;
-    att_combine<OP_NSPLIT>(sm, sl, o, mo, lo, oo);
-    emit(oo / lo);
-  }
-  if (fused) oproj();
-}
-
-// The rows of op_attn_kernel launched with nsplit > 1: the eight split states of (row, head)
-// combined in split order (wave 0), then (opart) the head's O projection by all eight waves.
-template <int FMT>
-__global__ __launch_bounds__(64 * ILL_WAVES) void op_attn_combine_kernel(OpCtx c, const float* scratch, OpMat Wo, float* opart,
-                                                                       int M) {
-  __shared__ _Float16 aoh[64];
-  const int done = gld(&c.st->done);
-  const int rh = blockIdx.x, w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int t = rh / ILL_NH, h = rh % ILL_NH;
-  // with opart (q8 / f16) the head's O projection follows, as in op_attn_kernel
-  constexpr bool OFUSE = FMT != 2;
-  const bool fused = OFUSE && opart != nullptr;
-  ORows<OFUSE ? FMT : 1> orw;
-  if constexpr (OFUSE)
-    if (fused) orows_fetch<FMT>(Wo, h, w, lane, orw);
-  if (w == 0) {
-    float m[OP_NSPLIT], l[OP_NSPLIT], o[OP_NSPLIT];
-#pragma unroll
-    for (int s = 0; s < OP_NSPLIT; s++) {
-      const float* src = scratch + ((size_t)rh * OP_NSPLIT + s) * OP_SPLIT_W;
-      m[s] = gld(src);
-      l[s] = gld(src + 1);
-      o[s] = gld(src + 2 + lane);
-    }
-    float mo, lo, oo;
-    att_combine<OP_NSPLIT>(m, l, o, mo, lo, oo);
-    const __half hv = __float2half(oo / lo);
-    if (fused) aoh[lane] = (_Float16)hv;
-    else if (!done) gst((uint16_t*)(c.ao + (size_t)t * ILL_H + h * 64 + lane), (uint16_t)__half_as_ushort(hv));
-  }
-  if constexpr (OFUSE)
-    if (fused) {
-      __syncthreads();
-      orows_apply<FMT>(orw, aoh, w, lane, opart + ((size_t)h * M + t) * ILL_H);
-    }
-}
-
 // ---- attention of prefill chunks (more than 16 rows): MFMA flash attention --------------
 // One workgroup of OP_RW waves per (16-row block, query head h): chunk c goes to wave
 // c % OP_RW, which folds its chunks in order, and the waves' states are combined at the end
@@ -1394,13 +661,13 @@ __global__ __launch_bounds__(64 * ILL_WAVES) void op_attn_combine_kernel(OpCtx c
 // reads, and its 4 kg groups' writes, on the same banks)
 #define OP_PLD 68
 template <bool SWZ>   // the K/V cache layout (ill_common.h): swizzled for q8 / f16, rows for q4
-__global__ __launch_bounds__(64 * OP_RW) void op_attn_rows_kernel(OpCtx c, int layer, int M) {
+__global__ __launch_bounds__(64 * OP_RW) void op_attn_rows_kernel(OpCtx c, int layer, int M, int blk0) {
   __shared__ __attribute__((aligned(16))) float pbw[OP_RW][16 * OP_PLD];
   __shared__ float sm_[OP_RW][16], sl_[OP_RW][16], so_[OP_RW][16][64];
   const OpHdr hd = op_hdr(c);
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, kg = lane >> 4, n = lane & 15;
   float* pb = pbw[w];
-  const int t0 = 16 * blockIdx.x, h = blockIdx.y, g = h / 7;
+  const int t0 = 16 * (blk0 + (int)blockIdx.x), h = blockIdx.y, g = h / 7;
   const int pos = hd.pos;
   // A operand: lane (kg, n) holds row t0 + n, dims 32 ks + 8 kg + i
   v8h qa[2][2];

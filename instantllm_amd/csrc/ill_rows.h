@@ -28,6 +28,12 @@
 #pragma once
 #include "ill_ops.h"
 
+// Prompt chunks of up to this many rows run on the row kernels (16-row groups in grid.y, each
+// reading the weights again), longer ones on the ring GEMMs, whose tiles share them. Whole
+// prompts, ms, row kernels / ring: q4 48 tokens 0.78 / 1.12, 100 1.11 / 1.20, 128 1.22 / 1.22,
+// 200 1.58 / 1.32; q8 100 1.10 / 1.23, 128 1.20 / 1.24, 200 1.52 / 1.33; f16 100 1.15 / 1.28,
+// 128 1.26 / 1.30, 200 1.60 / 1.34.
+#define ROW_MAXM 112
 #define ROW_SSQ 64      // floats per row of the sum-of-squares partials (56 tiles, then zeros)
 #define ROW_NSPLIT 8    // attention splits of a row: chunk c to split (c / 8) % 8, wave c % 8
 #define ROW_ST 72       // floats per (row, head, split) state: o[64], m, l
@@ -36,14 +42,16 @@
 // 16 kg .. + 15 (the tiled layout, op_wt_off: 1 KB (q8) or two runs of 1 KB (f16) per wave).
 template <int FMT>
 struct RowB {
-  uint4 q[FMT == 0 ? 2 : 1];
-  uint16_t s;   // q8: the scale
+  std::conditional_t<FMT == 2, uint2, uint4> q[FMT == 0 ? 2 : 1];
+  std::conditional_t<FMT == 2, uint32_t, uint16_t> s;   // q8: the scale; q4: (scale, min)
 };
 template <int FMT>
 __device__ __forceinline__ void row_fetch(const OpMat& W, int tile, int ks, int lane, RowB<FMT>& b) {
-  static_assert(FMT != 2, "q8 / f16");
   const int blk = (tile >> 3) * (W.K >> 6) + ks, sub = tile & 7;
-  if constexpr (FMT == 1) {
+  if constexpr (FMT == 2) {
+    b.q[0] = gld((const uint2*)(W.w + ((size_t)blk * 8 + sub) * 512) + lane);
+    b.s = gld((const uint32_t*)W.s + (size_t)blk * 128 + sub * 16 + (lane & 15));
+  } else if constexpr (FMT == 1) {
     b.q[0] = gld((const uint4*)(W.w + ((size_t)blk * 8 + sub) * 1024) + lane);
     const int per = 64 / W.qg;
     b.s = gld(W.s + ((size_t)blk * 128 + sub * 16 + (lane & 15)) * per + (per == 2 ? lane >> 5 : 0));
@@ -56,15 +64,22 @@ __device__ __forceinline__ void row_fetch(const OpMat& W, int tile, int ks, int 
 // columns 16 kg + 8 e .. + 7 as the MFMA operand
 template <int FMT>
 __device__ __forceinline__ v8h row_vals(const RowB<FMT>& b, int e) {
-  if constexpr (FMT == 0) return u4_to_v8h(b.q[e]);
-  v8h o;
-  _Float16 h[8];
-  const _Float16 sc = (_Float16)h2f(b.s);
-  op_q8x4(e == 0 ? b.q[0].x : b.q[0].z, sc, h);
-  op_q8x4(e == 0 ? b.q[0].y : b.q[0].w, sc, h + 4);
+  if constexpr (FMT == 0) {
+    return u4_to_v8h(b.q[e]);
+  } else {
+    v8h o;
+    _Float16 h[8];
+    if constexpr (FMT == 2) {
+      op_q4x8(e == 0 ? b.q[0].x : b.q[0].y, (_Float16)h2f(b.s & 0xffff), (_Float16)h2f(b.s >> 16), h);
+    } else {
+      const _Float16 sc = (_Float16)h2f(b.s);
+      op_q8x4(e == 0 ? b.q[0].x : b.q[0].z, sc, h);
+      op_q8x4(e == 0 ? b.q[0].y : b.q[0].w, sc, h + 4);
+    }
 #pragma unroll
-  for (int i = 0; i < 8; i++) o[i] = h[i];
-  return o;
+    for (int i = 0; i < 8; i++) o[i] = h[i];
+    return o;
+  }
 }
 
 // the rows a lane's operand and results hold: operand row n, result rows 4 kg + r
@@ -190,6 +205,7 @@ __global__ __launch_bounds__(448) void row_qkv_kernel(OpCtx c, OpMat W, const fl
 // One chunk per wave up to 4096 positions; 512 positions of 1 row take 2 workgroups.
 // A tree pass's positions from pos on live in the slots of the row's ancestors (slot pos + row):
 // K rows are loaded from those slots, V rows of such a chunk are patched in LDS.
+template <bool SWZ>   // the K/V cache layout (ill_common.h): swizzled for q8 / f16, rows for q4
 __global__ __launch_bounds__(64 * ILL_WAVES) void row_attn_kernel(OpCtx c, int layer, int M, int nsplit, float* att) {
   __shared__ float cm[ILL_WAVES][8], cl[ILL_WAVES][8];
   __shared__ __attribute__((aligned(16))) float co[ILL_WAVES][7][68];
@@ -212,14 +228,14 @@ __global__ __launch_bounds__(64 * ILL_WAVES) void row_attn_kernel(OpCtx c, int l
   uint4 kf[4][2], vf[4][2];
   auto kload = [&](int b, int slot) {
 #pragma unroll
-    for (int ks = 0; ks < 2; ks++) kf[b][ks] = gld((const uint4*)(kb + kv_k_off(slot, 32 * ks + 8 * kg, true)));
+    for (int ks = 0; ks < 2; ks++) kf[b][ks] = gld((const uint4*)(kb + kv_k_off(slot, 32 * ks + 8 * kg, SWZ)));
   };
   auto kkey = [&](int b) { return 32 * (b >> 1) + 8 * (n >> 2) + 4 * (b & 1) + (n & 3); };
   auto vload = [&](int ch) {
 #pragma unroll
     for (int nb = 0; nb < 4; nb++)
 #pragma unroll
-      for (int s = 0; s < 2; s++) vf[nb][s] = gld((const uint4*)(vb + kv_v_off(64 * ch + 32 * s + 8 * kg, 16 * nb + n, true)));
+      for (int s = 0; s < 2; s++) vf[nb][s] = gld((const uint4*)(vb + kv_v_off(64 * ch + 32 * s + 8 * kg, 16 * nb + n, SWZ)));
   };
   // the first chunk at its plain slots, before the header is waited for
   {
@@ -280,7 +296,7 @@ __global__ __launch_bounds__(64 * ILL_WAVES) void row_attn_kernel(OpCtx c, int l
         uint16_t pv[16];
 #pragma unroll
         for (int k = 0; k < 16; k++)
-          if (p0 + k < p1) pv[k] = gld(vb + kv_v_off(slot_of(64 * ch + p0 + k), lane, true));
+          if (p0 + k < p1) pv[k] = gld(vb + kv_v_off(slot_of(64 * ch + p0 + k), lane, SWZ));
 #pragma unroll
         for (int k = 0; k < 16; k++)
           if (p0 + k < p1) vr[lane * 72 + p0 + k] = pv[k];
@@ -389,78 +405,94 @@ __global__ __launch_bounds__(64 * ILL_WAVES) void row_attn_kernel(OpCtx c, int l
 // O projection: a workgroup per 16 output columns, seven waves of two k-steps (= heads) each.
 // Wave w combines the split states of its heads (lane: head 2 w + lane / 32, dims 2 (lane % 32),
 // + 1) into their f16 outputs. nsplit: the splits the host expects (loaded before the header is
-// waited for; a longer row's others follow).
-template <int FMT, int MT>
+// waited for; a longer row's others follow). AO: rows m0 .. of a prompt, their f16 attention
+// outputs in c.ao.
+template <int FMT, int MT, bool AO>
 __global__ __launch_bounds__(448) void row_o_kernel(OpCtx c, OpMat W, const float* att, float* ssq, int M, int nsplit) {
-  __shared__ __attribute__((aligned(16))) _Float16 As[7][MT][136];
+  __shared__ __attribute__((aligned(16))) _Float16 As[AO ? 1 : 7][AO ? 1 : MT][136];
   __shared__ float red[7][MT * 16];
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, kg = lane >> 4, n = lane & 15;
-  const int tile = blockIdx.x, Mg = M;
+  const int tile = blockIdx.x, m0 = AO ? 16 * blockIdx.y : 0, Mg = min(M - m0, MT);
   const OpHdr hd = op_hdr(c);
-  const int h = 2 * w + (lane >> 5), d2 = 2 * (lane & 31);
-  const float* st0 = att + (size_t)h * ROW_NSPLIT * ROW_ST;
-  constexpr int MB = MT < 4 ? MT : 4;   // rows combined per round
-  float2 o[MB][ROW_NSPLIT], q[MB][ROW_NSPLIT];   // (o of the two dims), (m, l)
-  auto states = [&](int r0, int s0, int s1) {   // the states s0 <= s < s1 of rows r0 ..
-#pragma unroll
-    for (int m = 0; m < MB; m++) {
-      const float* src = st0 + (size_t)min(r0 + m, Mg - 1) * ILL_NH * ROW_NSPLIT * ROW_ST;
-#pragma unroll
-      for (int s = 0; s < ROW_NSPLIT; s++)
-        if (s >= s0 && s < s1) {
-          o[m][s] = gld((const float2*)(src + s * ROW_ST + d2));
-          q[m][s] = gld((const float2*)(src + s * ROW_ST + 64));
-        }
-    }
-  };
-  states(0, 0, nsplit);
   RowB<FMT> wb[2];
-#pragma unroll
-  for (int s = 0; s < 2; s++) row_fetch<FMT>(W, tile, 2 * w + s, lane, wb[s]);
+  float ex;
   const int em = min(tid >> 4, MT - 1), ei = tid & 15;
-  const float ex = gld(c.x + (size_t)min(em, Mg - 1) * ILL_H + 16 * tile + ei);
-  const int dp = gld(c.tree + ILL_TR_DEPTH + n);
-  __builtin_amdgcn_sched_barrier(0);
-  auto splits = [&](int m) {   // of row m
-    const int dep = hd.mode == ILL_MODE_TREE ? __builtin_amdgcn_readlane(dp, m) : (hd.mode == ILL_MODE_DECODE ? 0 : m);
-    return __builtin_amdgcn_readfirstlane(min(ROW_NSPLIT, (((hd.pos + dep + 64) >> 6) + 7) >> 3));
+  auto fetch = [&]() {
+#pragma unroll
+    for (int s = 0; s < 2; s++) row_fetch<FMT>(W, tile, 2 * w + s, lane, wb[s]);
+    ex = gld(c.x + (size_t)(m0 + min(em, Mg - 1)) * ILL_H + 16 * tile + ei);
   };
-  const int smax = __builtin_amdgcn_readfirstlane(min(ROW_NSPLIT, (((hd.pos + MT + 63) >> 6) + 7) >> 3));
-  if (smax > nsplit) states(0, nsplit, smax);
+  uint4 av[AO ? 4 : 1];
+  if constexpr (AO) {
+    const uint4* ar = (const uint4*)(c.ao + (size_t)(m0 + min(n, Mg - 1)) * ILL_H + 128 * w);
+#pragma unroll
+    for (int i = 0; i < 4; i++) av[i] = gld(ar + 8 * (i >> 1) + 2 * kg + (i & 1));
+    fetch();
+    __builtin_amdgcn_sched_barrier(0);
+  } else {
+    const int h = 2 * w + (lane >> 5), d2 = 2 * (lane & 31);
+    const float* st0 = att + (size_t)h * ROW_NSPLIT * ROW_ST;
+    constexpr int MB = MT < 4 ? MT : 4;   // rows combined per round
+    float2 o[MB][ROW_NSPLIT], q[MB][ROW_NSPLIT];   // (o of the two dims), (m, l)
+    auto states = [&](int r0, int s0, int s1) {   // the states s0 <= s < s1 of rows r0 ..
+#pragma unroll
+      for (int m = 0; m < MB; m++) {
+        const float* src = st0 + (size_t)min(r0 + m, Mg - 1) * ILL_NH * ROW_NSPLIT * ROW_ST;
+#pragma unroll
+        for (int s = 0; s < ROW_NSPLIT; s++)
+          if (s >= s0 && s < s1) {
+            o[m][s] = gld((const float2*)(src + s * ROW_ST + d2));
+            q[m][s] = gld((const float2*)(src + s * ROW_ST + 64));
+          }
+      }
+    };
+    states(0, 0, nsplit);
+    fetch();
+    const int dp = gld(c.tree + ILL_TR_DEPTH + n);
+    __builtin_amdgcn_sched_barrier(0);
+    auto splits = [&](int m) {   // of row m
+      const int dep = hd.mode == ILL_MODE_TREE ? __builtin_amdgcn_readlane(dp, m) : (hd.mode == ILL_MODE_DECODE ? 0 : m);
+      return __builtin_amdgcn_readfirstlane(min(ROW_NSPLIT, (((hd.pos + dep + 64) >> 6) + 7) >> 3));
+    };
+    const int smax = __builtin_amdgcn_readfirstlane(min(ROW_NSPLIT, (((hd.pos + MT + 63) >> 6) + 7) >> 3));
+    if (smax > nsplit) states(0, nsplit, smax);
 #pragma unroll 1
-  for (int r0 = 0; r0 < MT; r0 += MB) {
-    if (r0 > 0) {
-      if (r0 >= Mg) break;
-      states(r0, 0, smax);
+    for (int r0 = 0; r0 < MT; r0 += MB) {
+      if (r0 > 0) {
+        if (r0 >= Mg) break;
+        states(r0, 0, smax);
+      }
+#pragma unroll
+      for (int m = 0; m < MB; m++) {
+        const int nne = splits(min(r0 + m, Mg - 1));
+        float mm = q[m][0].x;
+#pragma unroll
+        for (int s = 1; s < ROW_NSPLIT; s++)
+          if (s < nne) mm = fmaxf(mm, q[m][s].x);
+        float l = 0.f, a0 = 0.f, a1 = 0.f;
+#pragma unroll
+        for (int s = 0; s < ROW_NSPLIT; s++)
+          if (s < nne) {
+            const float e = att_exp(q[m][s].x - mm);
+            l = l + q[m][s].y * e;
+            a0 = a0 + o[m][s].x * e;
+            a1 = a1 + o[m][s].y * e;
+          }
+        _Float16* d = &As[w][r0 + m][2 * lane];   // k-step lane / 32, column 2 (lane % 32)
+        d[0] = (_Float16)__float2half(a0 / l);
+        d[1] = (_Float16)__float2half(a1 / l);
+      }
     }
-#pragma unroll
-    for (int m = 0; m < MB; m++) {
-      const int nne = splits(min(r0 + m, Mg - 1));
-      float mm = q[m][0].x;
-#pragma unroll
-      for (int s = 1; s < ROW_NSPLIT; s++)
-        if (s < nne) mm = fmaxf(mm, q[m][s].x);
-      float l = 0.f, a0 = 0.f, a1 = 0.f;
-#pragma unroll
-      for (int s = 0; s < ROW_NSPLIT; s++)
-        if (s < nne) {
-          const float e = att_exp(q[m][s].x - mm);
-          l = l + q[m][s].y * e;
-          a0 = a0 + o[m][s].x * e;
-          a1 = a1 + o[m][s].y * e;
-        }
-      _Float16* d = &As[w][r0 + m][2 * lane];   // k-step lane / 32, column 2 (lane % 32)
-      d[0] = (_Float16)__float2half(a0 / l);
-      d[1] = (_Float16)__float2half(a1 / l);
-    }
+    row_wave_sync();
   }
-  row_wave_sync();
   v4f acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int s = 0; s < 2; s++)
 #pragma unroll
     for (int e = 0; e < 2; e++) {
-      const v8h a = *(const v8h*)&As[w][row_a<MT>(n)][64 * s + 16 * kg + 8 * e];
+      v8h a;
+      if constexpr (AO) a = u4_to_v8h(av[2 * s + e]);
+      else a = *(const v8h*)&As[w][row_a<MT>(n)][64 * s + 16 * kg + 8 * e];
       acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, row_vals<FMT>(wb[s], e), acc, 0, 0, 0);
     }
   row_put<MT>(red[w], acc, kg, n);
@@ -469,7 +501,7 @@ __global__ __launch_bounds__(448) void row_o_kernel(OpCtx c, OpMat W, const floa
   float y = red[0][tid];
 #pragma unroll
   for (int i = 1; i < 7; i++) y += red[i][tid];
-  row_resid(c, ssq, em, tile, ei, ex, y);
+  row_resid(c, ssq, m0 + em, tile, ei, ex, y);
 }
 
 // Gate/up: a workgroup per four tiles (32 hidden units), a pair of waves per tile splitting K.

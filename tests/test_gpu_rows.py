@@ -82,3 +82,27 @@ def test_captured_step_replayed_at_a_longer_context(model):
             last = one(e, pos + i, t)
         assert np.array_equal(last, graph), pos
         e.kv_copy_in(k, v)
+
+
+@pytest.mark.parametrize("fmt", [F.FMT_Q4, F.FMT_Q8, F.FMT_F16], ids=["q4", "q8", "f16"])
+def test_prompts_at_the_row_kernels_edges(fmt, tmp_path):
+    """Prompt chunks around the longest one the row kernels take (112 rows) and its 16-row
+    groups, a 1-row last chunk (513 = 512 + 1), and prompts in two calls whose second one is
+    short: last-row logits against the oracle."""
+    from instantllm_amd.engine import Engine
+    path = str(tmp_path / "m.ill")
+    synth.build_model(path, fmt, seed=6, shape=synth.ModelShape(layers=2, vocab=VOCAB))
+    m = qwen.Model(illread.load(path))
+    e = Engine(path, max_context=1024, max_pass=16, max_steps=64)
+    toks = [int(t) for t in np.random.default_rng(700 + fmt).integers(0, VOCAB, size=600)]
+    try:
+        for parts in ((17,), (80,), (111,), (112,), (113,), (128,), (513,), (150, 16), (150, 17), (200, 97), (20, 1, 3)):
+            e.set_state(pos=0, n=1, maxsteps=64, eos=NO_EOS)
+            n = 0
+            for k in parts:
+                e.prefill(toks[n:n + k], write_logits=True)
+                n += k
+            ref = m.forward(toks[:n], m.new_cache(n + 1))
+            assert metrics.rel_l2(e.read_logits(0), ref) <= REL_L2_TOL, parts
+    finally:
+        e.close()
