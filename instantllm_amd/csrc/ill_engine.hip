@@ -398,21 +398,27 @@ void row_seq(ill_engine* e, int M, int lm_rows) {
   hipStream_t s = e->stream;
   const int mg = (M + 15) / 16;
   hipLaunchKernelGGL(row_embed_kernel<FMT>, dim3((M + 3) / 4), dim3(256), 0, s, c, e->ssq, M);
-  // up to 16 rows: one attention workgroup per (row, KV group) and 512 positions of the context
-  // the host expects (the result does not depend on the split)
+  // Up to 16 rows: attention workgroups per (row, KV group), by the context the host expects
+  // (the result does not depend on the split): one per 512 positions, but several rows stay
+  // unsplit up to 768 positions, where a second chunk for half of the waves costs less than the
+  // combining kernel (4 rows, q8, us per pass: 597 at 48 positions, unsplit 662 at 512 and 708 at
+  // 1000, split 692 at 2000).
   const int nch = (e->pos_hint + M + 63) / 64;
-  const int nsplit = std::max(1, std::min(ROW_NSPLIT, (nch + 7) / 8));
+  const int nsplit = M > 1 && nch <= 12 ? 1 : std::max(1, std::min(ROW_NSPLIT, (nch + 7) / 8));
   for (int l = 0; l < e->layers; l++) {
     const OpLayerW& L = e->holayers[l];
     hipLaunchKernelGGL((row_qkv_kernel<FMT, MT>), dim3(ILL_NQB, mg), dim3(448), 0, s, c, L.qkv, L.ln1, L.bqkv, e->ssq, l, M, e->pos_hint);
     if (M > 16) {
       if (l + 1 == e->layers) return op_last_row<FMT>(e, M, lm_rows);
       op_attn_rows<FMT>(e, l, M, 0);
-      if constexpr (MT == 16) hipLaunchKernelGGL((row_o_kernel<FMT, MT, true>), dim3(ILL_NOT, mg), dim3(448), 0, s, c, L.o, nullptr, e->ssq, M, 0);
     } else {
       hipLaunchKernelGGL(row_attn_kernel<FMT != 2>, dim3(M * ILL_NKV * nsplit), dim3(64 * ILL_WAVES), 0, s, c, l, M, nsplit, e->opart);
-      hipLaunchKernelGGL((row_o_kernel<FMT, MT, false>), dim3(ILL_NOT), dim3(448), 0, s, c, L.o, e->opart, e->ssq, M, nsplit);
+      if (M > 1 && nsplit > 1) hipLaunchKernelGGL(row_comb_kernel, dim3((M * ILL_NH + 3) / 4), dim3(256), 0, s, c, (const float*)e->opart, M);
     }
+    if (M == 1 && nsplit > 1)
+      hipLaunchKernelGGL((row_o_kernel<FMT, 1, false>), dim3(ILL_NOT), dim3(448), 0, s, c, L.o, (const float*)e->opart, e->ssq, M, nsplit);
+    else
+      hipLaunchKernelGGL((row_o_kernel<FMT, MT, true>), dim3(ILL_NOT, mg), dim3(448), 0, s, c, L.o, nullptr, e->ssq, M, 0);
     hipLaunchKernelGGL((row_gu_kernel<FMT, MT>), dim3(2 * ILL_FF / 64, mg), dim3(512), 0, s, c, L.gu, L.ln2, e->ssq, M);
     hipLaunchKernelGGL((row_down_kernel<FMT, MT>), dim3(ILL_NOT, mg), dim3(1024), 0, s, c, L.d, e->ssq, M);
   }

@@ -85,7 +85,7 @@ struct OpCtx {
   float* q;              // [M][896] queries
   __half* ao;            // [M][896] attention output
   __half* h;             // [M][4864] SiLU(gate) * up
-  uint64_t* amax;        // [V/128][16] argmax keys of the lm_head tiles
+  uint64_t* amax;        // [16][V/128] argmax keys of the lm_head tiles
   float* logits;         // [16][V]
   int maxctx, layers, vocab;
   int kvswz;             // K/V cache layout: 1 swizzled (q8 / f16), 0 rows (q4; ill_common.h)
@@ -364,7 +364,7 @@ __device__ __forceinline__ void op_gemm_epilogue(const OpGemmArgs& a, const OpHd
     if (tid < 16) {
       uint64_t k = red[0][tid];
       for (int ww = 1; ww < 4; ww++) k = red[ww][tid] > k ? red[ww][tid] : k;
-      c.amax[(size_t)blockIdx.x * 16 + tid] = k;
+      c.amax[(size_t)tid * gridDim.x + blockIdx.x] = k;
     }
   }
 }
@@ -806,30 +806,44 @@ __global__ __launch_bounds__(64 * OP_RW) void op_attn_rows_kernel(OpCtx c, int l
 __global__ __launch_bounds__(ILL_WG_THREADS) void op_commit_kernel(IllPassArgs a, const uint64_t* amax, int ntiles, int kvswz) {
   __shared__ PassHdr H;
   __shared__ CommitLds C;
-  __shared__ uint64_t best[ILL_WAVES];
-  load_hdr(a, H);
-  if (H.done) return;
+  __shared__ uint64_t best[16][ILL_WAVES];
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
   int stopreq = 0;   // the host's stop word (see ill_pass_kernel), waited for at the commit
   if (tid == 0 && a.stop_host) stopreq = __hip_atomic_load((const GAS int32_t*)a.stop_host, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-  for (int t = H.lmh0; t < H.lmh0 + H.lmhn; t++) {
+  load_hdr(a, H);
+  if (H.done) return;
+  // the greatest key of a wave's lanes: the values first, then the lowest index among them
+  auto wmax = [&](uint64_t k) {
+    const uint32_t hi = (uint32_t)(k >> 32), m = group_reduce<64>(hi, OpMaxU{});
+    return ((uint64_t)m << 32) | group_reduce<64>(hi == m ? (uint32_t)k : 0u, OpMaxU{});
+  };
+  auto of_row = [&](int t, int i0, int step) {   // tiles i0, i0 + step, .. of row t, four at a time
+    const uint64_t* r = amax + (size_t)t * ntiles;
     uint64_t k = 0;
-    for (int i = tid; i < ntiles; i += ILL_WG_THREADS) {
-      const uint64_t kk = amax[(size_t)i * 16 + t];
-      k = kk > k ? kk : k;
+    for (int i = i0; i < ntiles; i += 4 * step) {
+      uint64_t v[4];
+#pragma unroll
+      for (int u = 0; u < 4; u++) v[u] = gld(r + min(i + u * step, ntiles - 1));
+#pragma unroll
+      for (int u = 0; u < 4; u++) k = v[u] > k ? v[u] : k;
     }
-    for (int o = 32; o >= 1; o >>= 1) {
-      const uint64_t ok = __shfl_xor(k, o, 64);
-      k = ok > k ? ok : k;
-    }
-    if (lane == 0) best[w] = k;
-    __syncthreads();
-    if (tid == 0) {
-      uint64_t m = best[0];
-      for (int i = 1; i < ILL_WAVES; i++) m = best[i] > m ? best[i] : m;
-      C.g[t] = (int)(0xFFFFFFFFu - (uint32_t)(m & 0xFFFFFFFFu));
-    }
-    __syncthreads();
+    return wmax(k);
+  };
+  // one row: its tiles over all waves; more: a row per wave (16 rows: 25 us of commit with the
+  // rows one after the other, each over all waves and through two barriers)
+  const bool split = H.lmhn == 1;
+  for (int t = H.lmh0 + (split ? 0 : w); t < H.lmh0 + H.lmhn; t += split ? 1 : ILL_WAVES) {
+    const uint64_t k = split ? of_row(t, tid, ILL_WG_THREADS) : of_row(t, lane, 64);
+    if (lane == 0) best[t][split ? w : 0] = k;
   }
+  __syncthreads();
+  if (tid < H.lmhn) {
+    const int t = H.lmh0 + tid;
+    uint64_t m = best[t][0];
+    if (split)
+      for (int i = 1; i < ILL_WAVES; i++) m = best[t][i] > m ? best[t][i] : m;
+    C.g[t] = (int)(0xFFFFFFFFu - (uint32_t)(m & 0xFFFFFFFFu));
+  }
+  __syncthreads();
   commit_apply(a, H, C, false, stopreq, kvswz != 0);
 }

@@ -194,6 +194,29 @@ __global__ __launch_bounds__(448) void row_qkv_kernel(OpCtx c, OpMat W, const fl
   epi_qkv(c, hd, layer, m0 + em, b, ei, x0, x1, ep, cs, eb);
 }
 
+// A row's output in two dims from its split states (o of the two dims; m, l), in split order.
+__device__ __forceinline__ void row_combine(const float2* o, const float2* ml, int nne, float& y0, float& y1) {
+  float mm = ml[0].x;
+#pragma unroll
+  for (int s = 1; s < ROW_NSPLIT; s++)
+    if (s < nne) mm = fmaxf(mm, ml[s].x);
+  float l = 0.f, a0 = 0.f, a1 = 0.f;
+#pragma unroll
+  for (int s = 0; s < ROW_NSPLIT; s++)
+    if (s < nne) {
+      const float e = att_exp(ml[s].x - mm);
+      l = l + ml[s].y * e;
+      a0 = a0 + o[s].x * e;
+      a1 = a1 + o[s].y * e;
+    }
+  y0 = a0 / l;
+  y1 = a1 / l;
+}
+// the splits of a row at pos + dep
+__device__ __forceinline__ int row_splits(int pos, int dep) {
+  return __builtin_amdgcn_readfirstlane(min(ROW_NSPLIT, (((pos + dep + 64) >> 6) + 7) >> 3));
+}
+
 // Attention: a workgroup per (row, KV group, split j < nsplit) takes the splits j, j + nsplit, ..;
 // wave w evaluates chunk 8 s + w (64 positions; then every 64th chunk) of split s for the
 // group's seven heads at once: the heads are columns of the MFMA blocks (scores: K rows x heads,
@@ -201,8 +224,10 @@ __global__ __launch_bounds__(448) void row_qkv_kernel(OpCtx c, OpMat W, const fl
 // P needs no cross-lane move (the key of block b, row 4 kg + r is 32 (b / 2) + 8 kg + 4 (b % 2) + r,
 // so a lane's scores are the eight consecutive keys of its operand slots). q and P are split into
 // f16 high and low parts (fp32-accurate products). The waves' states are combined in wave order
-// into the split's state; row_o_kernel combines the splits.
-// One chunk per wave up to 4096 positions; 512 positions of 1 row take 2 workgroups.
+// into the split's state, the row's splits in split order: here with nsplit = 1 (c.ao gets the
+// f16 output), else by the readers of att (row_o_kernel for one row, row_comb_kernel), with the
+// same arithmetic, so the launch's split does not change the result.
+// One chunk per wave up to 512 nsplit positions; 512 positions of 1 row take 2 workgroups.
 // A tree pass's positions from pos on live in the slots of the row's ancestors (slot pos + row):
 // K rows are loaded from those slots, V rows of such a chunk are patched in LDS.
 template <bool SWZ>   // the K/V cache layout (ill_common.h): swizzled for q8 / f16, rows for q4
@@ -211,6 +236,7 @@ __global__ __launch_bounds__(64 * ILL_WAVES) void row_attn_kernel(OpCtx c, int l
   __shared__ __attribute__((aligned(16))) float co[ILL_WAVES][7][68];
   __shared__ int path[ILL_WAVES][16];
   __shared__ __attribute__((aligned(16))) uint16_t vst[2][64 * 72];   // (pass rows span two chunks at most)
+  __shared__ float so[ROW_NSPLIT][7][64], sml[ROW_NSPLIT][7][2];      // nsplit 1: the splits' states
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, kg = lane >> 4, n = lane & 15;
   const int j = blockIdx.x % nsplit, g = (blockIdx.x / nsplit) % ILL_NKV, t = blockIdx.x / (nsplit * ILL_NKV);
   const float* qr = c.q + (size_t)t * ILL_H + (7 * g + min(n, 6)) * 64 + 8 * kg;
@@ -394,22 +420,69 @@ __global__ __launch_bounds__(64 * ILL_WAVES) void row_attn_kernel(OpCtx c, int l
       }
       float mo, lo, oo;
       att_combine<ILL_WAVES>(m, l, o, mo, lo, oo);
-      float* dst = att + (((size_t)t * ILL_NH + 7 * g + w) * ROW_NSPLIT + s) * ROW_ST;
-      gst(dst + lane, oo);
-      if (lane < 2) gst(dst + 64 + lane, lane == 0 ? mo : lo);
+      if (nsplit > 1) {
+        float* dst = att + (((size_t)t * ILL_NH + 7 * g + w) * ROW_NSPLIT + s) * ROW_ST;
+        gst(dst + lane, oo);
+        if (lane < 2) gst(dst + 64 + lane, lane == 0 ? mo : lo);
+      } else {
+        if (nne > 1) {
+          so[s][w][lane] = oo;
+          if (lane < 2) sml[s][w][lane] = lane == 0 ? mo : lo;
+        }
+        if (s + 1 == nne) {
+          float l = lo, a0 = oo;
+          if (nne > 1) {   // as row_combine, from LDS (this wave wrote the states)
+            row_wave_sync();
+            float mm = sml[0][w][0];
+#pragma unroll 1
+            for (int i = 1; i < nne; i++) mm = fmaxf(mm, sml[i][w][0]);
+            l = a0 = 0.f;
+#pragma unroll 1
+            for (int i = 0; i < nne; i++) {
+              const float e = att_exp(sml[i][w][0] - mm);
+              l = l + sml[i][w][1] * e;
+              a0 = a0 + so[i][w][lane] * e;
+            }
+          }
+          const float y = a0 / l;
+          gst((uint16_t*)(c.ao + (size_t)t * ILL_H + (7 * g + w) * 64 + lane), (uint16_t)__half_as_ushort(__float2half(y)));
+        }
+      }
     }
     if (s + nsplit < nne) lds_barrier();   // the states are read before the next split's are written
   }
 }
 
+// The split states of (row, head) pairs of passes of several rows, a wave per pair (lane: a
+// dim), into c.ao.
+__global__ __launch_bounds__(256) void row_comb_kernel(OpCtx c, const float* att, int M) {
+  const int lane = threadIdx.x & 63, rh = 4 * blockIdx.x + (threadIdx.x >> 6);
+  if (rh >= M * ILL_NH) return;
+  const int t = rh / ILL_NH;
+  const OpHdr hd = op_hdr(c);
+  const int dp = gld(c.tree + ILL_TR_DEPTH + min(t, 15));
+  const float* src = att + (size_t)rh * ROW_NSPLIT * ROW_ST;
+  float2 o[ROW_NSPLIT], ml[ROW_NSPLIT];
+#pragma unroll
+  for (int s = 0; s < ROW_NSPLIT; s++) {   // (states past the row's splits are not used)
+    o[s].x = gld(src + s * ROW_ST + lane);
+    ml[s] = gld((const float2*)(src + s * ROW_ST + 64));
+  }
+  const int dep = hd.mode == ILL_MODE_TREE ? dp : (hd.mode == ILL_MODE_DECODE ? 0 : t);
+  float y, unused;
+  row_combine(o, ml, row_splits(hd.pos, dep), y, unused);
+  if (!hd.done) gst((uint16_t*)(c.ao + (size_t)rh * 64 + lane), (uint16_t)__half_as_ushort(__float2half(y)));
+}
+
 // O projection: a workgroup per 16 output columns, seven waves of two k-steps (= heads) each.
-// Wave w combines the split states of its heads (lane: head 2 w + lane / 32, dims 2 (lane % 32),
-// + 1) into their f16 outputs. nsplit: the splits the host expects (loaded before the header is
-// waited for; a longer row's others follow). AO: rows m0 .. of a prompt, their f16 attention
-// outputs in c.ao.
+// AO: rows m0 .., their f16 attention outputs in c.ao. Else one row from its split states: wave w
+// combines those of its heads (lane: head 2 w + lane / 32, dims 2 (lane % 32), + 1). nsplit: the
+// splits the host expects (loaded before the header is waited for; a longer row's others
+// follow). Combining every row's states here as well took 16 us per layer at 16 rows (each of the
+// 56 workgroups repeats it) against 4 + 3 with row_comb_kernel.
 template <int FMT, int MT, bool AO>
 __global__ __launch_bounds__(448) void row_o_kernel(OpCtx c, OpMat W, const float* att, float* ssq, int M, int nsplit) {
-  __shared__ __attribute__((aligned(16))) _Float16 As[AO ? 1 : 7][AO ? 1 : MT][136];
+  __shared__ __attribute__((aligned(16))) _Float16 As[AO ? 1 : 7][1][136];
   __shared__ float red[7][MT * 16];
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, kg = lane >> 4, n = lane & 15;
   const int tile = blockIdx.x, m0 = AO ? 16 * blockIdx.y : 0, Mg = min(M - m0, MT);
@@ -422,6 +495,7 @@ __global__ __launch_bounds__(448) void row_o_kernel(OpCtx c, OpMat W, const floa
     for (int s = 0; s < 2; s++) row_fetch<FMT>(W, tile, 2 * w + s, lane, wb[s]);
     ex = gld(c.x + (size_t)(m0 + min(em, Mg - 1)) * ILL_H + 16 * tile + ei);
   };
+  static_assert(AO || MT == 1, "several rows: from c.ao");
   uint4 av[AO ? 4 : 1];
   if constexpr (AO) {
     const uint4* ar = (const uint4*)(c.ao + (size_t)(m0 + min(n, Mg - 1)) * ILL_H + 128 * w);
@@ -432,57 +506,26 @@ __global__ __launch_bounds__(448) void row_o_kernel(OpCtx c, OpMat W, const floa
   } else {
     const int h = 2 * w + (lane >> 5), d2 = 2 * (lane & 31);
     const float* st0 = att + (size_t)h * ROW_NSPLIT * ROW_ST;
-    constexpr int MB = MT < 4 ? MT : 4;   // rows combined per round
-    float2 o[MB][ROW_NSPLIT], q[MB][ROW_NSPLIT];   // (o of the two dims), (m, l)
-    auto states = [&](int r0, int s0, int s1) {   // the states s0 <= s < s1 of rows r0 ..
+    float2 o[ROW_NSPLIT], q[ROW_NSPLIT];   // (o of the two dims), (m, l)
+    auto states = [&](int s0, int s1) {   // s0 <= s < s1
 #pragma unroll
-      for (int m = 0; m < MB; m++) {
-        const float* src = st0 + (size_t)min(r0 + m, Mg - 1) * ILL_NH * ROW_NSPLIT * ROW_ST;
-#pragma unroll
-        for (int s = 0; s < ROW_NSPLIT; s++)
-          if (s >= s0 && s < s1) {
-            o[m][s] = gld((const float2*)(src + s * ROW_ST + d2));
-            q[m][s] = gld((const float2*)(src + s * ROW_ST + 64));
-          }
-      }
+      for (int s = 0; s < ROW_NSPLIT; s++)
+        if (s >= s0 && s < s1) {
+          o[s] = gld((const float2*)(st0 + s * ROW_ST + d2));
+          q[s] = gld((const float2*)(st0 + s * ROW_ST + 64));
+        }
     };
-    states(0, 0, nsplit);
+    states(0, nsplit);
     fetch();
-    const int dp = gld(c.tree + ILL_TR_DEPTH + n);
+    const int dp = gld(c.tree + ILL_TR_DEPTH);
     __builtin_amdgcn_sched_barrier(0);
-    auto splits = [&](int m) {   // of row m
-      const int dep = hd.mode == ILL_MODE_TREE ? __builtin_amdgcn_readlane(dp, m) : (hd.mode == ILL_MODE_DECODE ? 0 : m);
-      return __builtin_amdgcn_readfirstlane(min(ROW_NSPLIT, (((hd.pos + dep + 64) >> 6) + 7) >> 3));
-    };
-    const int smax = __builtin_amdgcn_readfirstlane(min(ROW_NSPLIT, (((hd.pos + MT + 63) >> 6) + 7) >> 3));
-    if (smax > nsplit) states(0, nsplit, smax);
-#pragma unroll 1
-    for (int r0 = 0; r0 < MT; r0 += MB) {
-      if (r0 > 0) {
-        if (r0 >= Mg) break;
-        states(r0, 0, smax);
-      }
-#pragma unroll
-      for (int m = 0; m < MB; m++) {
-        const int nne = splits(min(r0 + m, Mg - 1));
-        float mm = q[m][0].x;
-#pragma unroll
-        for (int s = 1; s < ROW_NSPLIT; s++)
-          if (s < nne) mm = fmaxf(mm, q[m][s].x);
-        float l = 0.f, a0 = 0.f, a1 = 0.f;
-#pragma unroll
-        for (int s = 0; s < ROW_NSPLIT; s++)
-          if (s < nne) {
-            const float e = att_exp(q[m][s].x - mm);
-            l = l + q[m][s].y * e;
-            a0 = a0 + o[m][s].x * e;
-            a1 = a1 + o[m][s].y * e;
-          }
-        _Float16* d = &As[w][r0 + m][2 * lane];   // k-step lane / 32, column 2 (lane % 32)
-        d[0] = (_Float16)__float2half(a0 / l);
-        d[1] = (_Float16)__float2half(a1 / l);
-      }
-    }
+    const int nne = row_splits(hd.pos, hd.mode == ILL_MODE_TREE ? dp : 0);
+    if (nne > nsplit) states(nsplit, nne);
+    float y0, y1;
+    row_combine(o, q, nne, y0, y1);
+    _Float16* d = &As[w][0][2 * lane];   // k-step lane / 32, column 2 (lane % 32)
+    d[0] = (_Float16)__float2half(y0);
+    d[1] = (_Float16)__float2half(y1);
     row_wave_sync();
   }
   v4f acc = {0.f, 0.f, 0.f, 0.f};
