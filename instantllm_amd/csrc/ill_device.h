@@ -65,6 +65,8 @@ __device__ __forceinline__ uint64_t clk() { return wall_clock64(); }
 
 // Tag of the lm_head argmax partials of a pass.
 __device__ __forceinline__ uint32_t tagof_lmh(uint32_t epoch) { return epoch * 32u + 31u; }
+// Tag of the q words and chunk states that attention helpers exchange in layer l.
+__device__ __forceinline__ uint32_t tagof_help(uint32_t epoch, int l) { return epoch * 32u + (uint32_t)l + 1u; }
 
 // Records the first timeout code; every wait gives up once any is recorded.
 __device__ __forceinline__ void set_err(IllCtl* ctl, int code) {

@@ -120,7 +120,7 @@ struct ill_engine {
   float2* rope = nullptr;
   uint16_t* kc = nullptr;
   uint16_t* vt = nullptr;
-  uint64_t *acc = nullptr, *lmp = nullptr, *pub = nullptr;
+  uint64_t *acc = nullptr, *lmp = nullptr, *pub = nullptr, *hq = nullptr, *hs = nullptr;
   uint4* part = nullptr;   // 16-row passes: down-projection partials (ILL_PART_WORDS 16-byte words)
   size_t acc_bytes = 0;
   float* logits = nullptr;
@@ -280,6 +280,8 @@ int count_passes(ill_engine* e, int n) {
   HCK(hipMemsetAsync(e->pub, 0, (size_t)ILL_PUB_WORDS * 8, e->stream));
   HCK(hipMemsetAsync(e->part, 0, (size_t)ILL_PART_WORDS * 16, e->stream));
   HCK(hipMemsetAsync(e->lmp, 0, (size_t)ILL_WG * 16 * 2 * 8, e->stream));
+  HCK(hipMemsetAsync(e->hq, 0, (size_t)ILL_NH * 64 * 8, e->stream));
+  HCK(hipMemsetAsync(e->hs, 0, (size_t)ILL_NH * (e->maxctx / 64) * ILL_HELP_W * 8, e->stream));
   HCK(hipStreamSynchronize(e->stream));
   e->passes_since_clear = (uint64_t)n;
   return 0;
@@ -760,7 +762,8 @@ int ill_create(const char* path, int max_context, int max_pass, int max_steps, i
             dalloc((void**)&e->rope, (size_t)(e->maxctx + 16) * 32 * 8) && dalloc((void**)&e->kc, kvb) && dalloc((void**)&e->vt, kvb) &&
             dalloc((void**)&e->acc, e->acc_bytes) &&
             dalloc((void**)&e->lmp, (size_t)ILL_WG * 16 * 2 * 8) && dalloc((void**)&e->pub, (size_t)ILL_PUB_WORDS * 8) &&
-            dalloc((void**)&e->part, (size_t)ILL_PART_WORDS * 16) &&
+            dalloc((void**)&e->part, (size_t)ILL_PART_WORDS * 16) && dalloc((void**)&e->hq, (size_t)ILL_NH * 64 * 8) &&
+            dalloc((void**)&e->hs, (size_t)ILL_NH * (e->maxctx / 64) * ILL_HELP_W * 8) &&
             dalloc((void**)&e->logits, (size_t)16 * vocab * 4) &&
             dalloc((void**)&e->out_dev, (size_t)max_steps * 4);
   ok = ok && dalloc((void**)&e->dolayers, sizeof(OpLayerW) * layers) && dalloc((void**)&e->octx.x, (size_t)ILL_OP_MAXM * ILL_H * 4) &&
@@ -822,6 +825,8 @@ int ill_create(const char* path, int max_context, int max_pass, int max_steps, i
   a.lmp = e->lmp;
   a.pub = e->pub;
   a.part = e->part;
+  a.hq = e->hq;
+  a.hs = e->hs;
   a.logits = e->logits;
   a.out_dev = e->out_dev;
   a.out_host = e->out_host;
@@ -856,7 +861,7 @@ int ill_destroy(ill_engine* e) {
   if (e->gexec) hipGraphExecDestroy(e->gexec);
   if (e->graph) hipGraphDestroy(e->graph);
   void* bufs[] = {e->dweights, e->dlayers, e->st, e->ctl, e->ptoks, e->tree, e->rope, e->kc, e->vt, e->acc,
-                  e->lmp, e->pub, e->part, e->logits, e->out_dev, e->args.trace, e->oweights, e->dolayers, e->octx.x, e->octx.xn,
+                  e->lmp, e->pub, e->part, e->hq, e->hs, e->logits, e->out_dev, e->args.trace, e->oweights, e->dolayers, e->octx.x, e->octx.xn,
                   e->octx.q, e->octx.ao, e->octx.h, e->octx.amax, e->opart, e->ssq, e->dtab, e->dtflg, e->dreq};
   for (void* p : bufs)
     if (p) hipFree(p);

@@ -12,6 +12,8 @@
 //   GUD[ub]  (76 WGs, 64 hidden units each)
 //            x'_l = XA[l] -> RMSNorm -> gate/up rows -> SiLU * up -> down projection
 //            restricted to the 64 units (split K) -> adds into XB[l] (= x_{l+1})
+//   HELP     (1-row passes past 512 positions) the attention chunks that the ATT workgroup of
+//            a head has no wave for
 //   LMH      (all WGs) final RMSNorm -> tied lm_head tiles -> per-WG argmax partials
 //   COMMIT   (WG 0) argmax (ties -> lowest id), token record, state advance, tree accept,
 //            KV compaction, epoch advance
@@ -39,8 +41,11 @@
 #define ILL_NRED (ILL_RED_Q * ILL_MAXT)
 #define ILL_R_RED0 108       // 16-row passes: REDUCE WGs 108..235 (row r / 8, column eighth r % 8)
 #define ILL_R_ATT1 236       // 16-row passes: ATT WGs 236..249, rows 8-15 of head wg - 236
-#define ILL_R_IDLE0 92       // 1-row passes: WGs 92..255 have no layer role; each stages
+#define ILL_R_IDLE0 92       // 1-row passes: WGs 92..255 have no layer role but HELP; each stages
 #define ILL_LMH_PRE 16       // ILL_LMH_PRE lm_head tiles (two per wave) in its LDS meanwhile
+#define ILL_HELP_R 8         // 1-row passes: HELP WGs per head
+#define ILL_R_HELP0 96       // HELP WGs 96..207 (a multiple of the 8 XCDs)
+#define ILL_HELP_W 72        // words of a helper's chunk state: o[64], m, l (padded)
 
 struct IllPassArgs {
   IllWeights W;
@@ -64,6 +69,8 @@ struct IllPassArgs {
   const int32_t* prompt;   // [4 + ILL_OB_MAX]: count, -, -, -, the last <= 256 prompt tokens
   int32_t* spec_host;      // pinned host [2]: passes and accepted drafts of speculative commits
   const int32_t* stop_host;   // pinned host word: nonzero once the host asked queued passes to stop
+  uint64_t* hq;            // 1-row passes past 512 positions: [14][64] tagged q words of the layer in flight
+  uint64_t* hs;            // and [14][maxctx / 64][ILL_HELP_W] tagged chunk states (o[64], m, l) of the helpers
   int maxctx;
   int maxsteps;
   IllLayerW L0;            // L[0] again: the pass's first weight stage reads these pointers from
@@ -710,6 +717,8 @@ struct AttLds {
   uint4 ahi[4 * T], alo[4 * T];
   float2 dsc[T];
   float p1[T == 1 ? ILL_WAVES : 1][64];   // T = 1: the waves' P scratch, outside the union
+  float hq[T == 1 ? 2 : 1][64];           // T = 1, HELP: q of the layer (by layer parity)
+  int hok[2];
 };
 
 // Per-wave scratch [T][64] for a chunk's probabilities. At T = 1 it lies outside the region
@@ -1445,7 +1454,11 @@ __device__ __forceinline__ bool role_att(const IllPassArgs& a, const PassHdr& H,
   // Waves without a shared chunk: at T = 1 the wave of the partial pair fetches chunk ns; in
   // 16-row passes every wave evaluates chunk ns, which needs the cache if it holds positions
   // below pos.
-  const int cfirst = sj < ns ? sj : (T == 1 ? att_pair_chunk(H, ns, cmax, (sj - ns) & 7) : (64 * ns < pos ? ns : -1));
+  // Past 512 positions (T = 1) every wave evaluates one chunk: slot ns % 8 the partial one, the
+  // others their first; the HELP workgroups do the rest (collect below).
+  const bool help = T == 1 && ns >= ILL_WAVES;
+  const bool mine = sj < ns && !(help && sj == (ns & 7));   // T = 1: this wave evaluates chunk sj
+  const int cfirst = mine ? sj : (T == 1 ? att_pair_chunk(H, ns, cmax, (sj - ns) & 7) : (64 * ns < pos ? ns : -1));
   KVFrag f;
   int fc = -1;   // cache chunk held in f
   // The slot's first chunk streams in while the input is awaited: cache positions below pos
@@ -1529,6 +1542,10 @@ __device__ __forceinline__ bool role_att(const IllPassArgs& a, const PassHdr& H,
       if (head < ILL_NH) {
         A.q[t][d] = x0;
         A.q[t][d + 32] = x1;
+        if (T == 1 && ns >= ILL_WAVES) {
+          astore64(a.hq + h * 64 + d, mkw(x0, tagof_help(H.epoch, l)));
+          astore64(a.hq + h * 64 + d + 32, mkw(x1, tagof_help(H.epoch, l)));
+        }
       } else if (head < ILL_NH + ILL_NKV) {
         const uint32_t h0 = f2h(x0), h1 = f2h(x1);
         A.k[t][d] = (uint16_t)h0;
@@ -1608,28 +1625,64 @@ __device__ __forceinline__ bool role_att(const IllPassArgs& a, const PassHdr& H,
       M[j] = k.mn;
     }
   };
-  for (int c = sj; c < ns; c += ILL_WAVES) {
-    if (c != fc) {
-      kv_fetch(kbase, vbase, c, lane, f);
-      fc = c;
-    }
-    float mx[4], ls[4], o[4][4];
-    chunk_eval<T>(H, A, stage, f, c, false, 0, qa, mx, ls, o);
-    fold(mx, ls, o);
-  }
+  bool okh = true;
   if constexpr (T == 1) {
+    // the states of the slot's chunks c0, c0 + 8, .. < ns from the helpers, folded in order
+    auto collect = [&](int c0) {
+      const uint32_t tag = tagof_help(H.epoch, l);
+      for (int cb = c0; cb < ns && okh; cb += 4 * ILL_WAVES) {
+        uint64_t wv[4][6];
+        okh = wave_wait([&]() {
+          bool ok = true;
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            const int c = cb + ILL_WAVES * i;
+            if (c < ns) {
+              const uint64_t* src = a.hs + ((size_t)h * (a.maxctx / 64) + c) * ILL_HELP_W;
+#pragma unroll
+              for (int k = 0; k < 6; k++) {
+                wv[i][k] = aload64(src + (k < 4 ? 16 * k + n : 60 + k));
+                ok &= wok(wv[i][k], tag);
+              }
+            }
+          }
+          return ok;
+        }, a.ctl, 800 + l);
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+          if (cb + ILL_WAVES * i < ns) {
+            const AttScale k = att_scale(M[0], wval(wv[i][4]));
+#pragma unroll
+            for (int nb = 0; nb < 4; nb++) O[nb][0] = att_fold(O[nb][0], wval(wv[i][nb]), k);
+            Lw[0] = att_fold(Lw[0], wval(wv[i][5]), k);
+            M[0] = k.mn;
+          }
+      }
+    };
+    if (mine) {
+      float mx[4], ls[4], o[4][4];
+      chunk_eval<T>(H, A, stage, f, sj, false, 0, qa, mx, ls, o);
+      fold(mx, ls, o);
+      if (help) collect(sj + ILL_WAVES);
+    }
     // the one partial pair (chunk ns, row 0) belongs to slot ns % 8, whose wave folds it
     // into the slot state after the slot's shared chunks, as the combine would
     if (sj == (ns & 7)) {
-      if (ns != fc) {
-        kv_fetch(kbase, vbase, ns, lane, f);
-        fc = ns;
-      }
       float mx[4], ls[4], o[4][4];
       chunk_eval<T>(H, A, stage, f, ns, true, 0, qa, mx, ls, o);
+      if (help) collect(sj);
       fold(mx, ls, o);
     }
   } else {
+    for (int c = sj; c < ns; c += ILL_WAVES) {
+      if (c != fc) {
+        kv_fetch(kbase, vbase, c, lane, f);
+        fc = c;
+      }
+      float mx[4], ls[4], o[4][4];
+      chunk_eval<T>(H, A, stage, f, c, false, 0, qa, mx, ls, o);
+      fold(mx, ls, o);
+    }
     for (int c = ns; c <= cmax; c++) {
       const bool cache = 64 * c < pos;
       if (cache && c != fc) {
@@ -1710,6 +1763,69 @@ __device__ __forceinline__ bool role_att(const IllPassArgs& a, const PassHdr& H,
     wait_vm();
     trace_mark(a, ILL_TRL * l + 12);
   }
+  return okh;
+}
+
+// HELP (1-row passes, ns = pos / 64 >= 8 shared chunks): workgroup r of head h evaluates chunks
+// that the head's ATT workgroup would reach only in a second round of its eight waves: r >= 1
+// the chunks 8 r + w, then every 56th, r = 0 the first chunk of the slot that holds the partial
+// chunk. The wave's first chunk is fetched ahead; q comes from ATT as tagged words, the chunk's
+// (o, m, l) goes back the same way, and ATT folds the states in the order of its own loop: the
+// same values, whoever evaluates a chunk. ATT overwrites q only after it has every state of the
+// layer, so a helper with a chunk has read it by then.
+// A chunk in a further round cost the step 2.4 us (the second, 24 layers: 314 -> 372 us from
+// 448 to 512 positions) to 3.6 us per layer (600 us at 2000 positions, 922 at 4000): its K/V
+// come after the evaluation before it, and prefetching them cost the step 15 us everywhere.
+// With the helpers: 359 us at 512 positions, 391 at 1000, 421 at 2000, 476 at 4000 (the step at
+// 256 positions unchanged: 314 us). Pausing the watchers between layers and collecting eight
+// states per poll instead of four made no difference (474-477 us at 4000).
+template <int T>
+__device__ __forceinline__ bool role_help(const IllPassArgs& a, const PassHdr& H, AttLds<T>& A, int hr, uint8_t* stage) {
+  const int tid = tid_opaque(), w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int kg = lane >> 4;
+  // workgroup i runs on XCD i % 8: the seven heads of (r, g) share an XCD, whose L2 then fetches
+  // their chunks once
+  const int rg = (hr & 7) + 8 * (hr / 56), r = rg >> 1, g = rg & 1, h = 7 * g + (hr >> 3) % 7;
+  static_assert(ILL_HELP_R * ILL_NH == 112 && ILL_R_HELP0 % 8 == 0, "two (r, g) per XCD");
+  const int ns = H.pos >> 6;
+  if (ns < ILL_WAVES || (r > 0 && ILL_WAVES * r >= ns)) return true;   // (uniform)
+  const int c0 = r > 0 ? ILL_WAVES * r + w : (w == (ns & 7) ? w : ns), step = r > 0 ? ILL_WAVES * (ILL_HELP_R - 1) : ns;
+  for (int l = 0; l < a.W.layers; l++) {
+    const uint16_t* kbase = a.kc + ((size_t)l * ILL_NKV + g) * a.maxctx * 64;
+    const uint16_t* vbase = a.vt + ((size_t)l * ILL_NKV + g) * a.maxctx * 64;
+    const uint32_t tag = tagof_help(H.epoch, l);
+    KVFrag f;
+    if (c0 < ns) kv_fetch(kbase, vbase, c0, lane, f);
+    if (w == 0) {   // one watcher wave
+      uint64_t q;
+      const bool ok = wave_wait([&]() { q = aload64(a.hq + h * 64 + lane); return wok(q, tag); }, a.ctl, 830 + l);
+      A.hq[l & 1][lane] = wval(q) * 0.125f;
+      if (lane == 0) A.hok[l & 1] = ok;
+    }
+    lds_barrier();
+    if (!A.hok[l & 1]) return false;
+    v8h qa[2][2];   // as role_att
+#pragma unroll
+    for (int ks = 0; ks < 2; ks++) {
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+        const float v = A.hq[l & 1][32 * ks + 8 * kg + i];
+        const _Float16 hi = (_Float16)v;
+        qa[ks][0][i] = hi;
+        qa[ks][1][i] = (_Float16)(v - (float)hi);
+      }
+    }
+    for (int c = c0; c < ns; c += step) {
+      if (c != c0) kv_fetch(kbase, vbase, c, lane, f);
+      float mx[4], ls[4], o[4][4];
+      chunk_eval<T>(H, A, stage, f, c, false, 0, qa, mx, ls, o);
+      uint64_t* dst = a.hs + ((size_t)h * (a.maxctx / 64) + c) * ILL_HELP_W;
+      const float ov = kg == 0 ? o[0][0] : kg == 1 ? o[1][0] : kg == 2 ? o[2][0] : o[3][0];
+      astore64(dst + lane, mkw(ov, tag));
+      if (lane < 2) astore64(dst + 64 + lane, mkw(lane == 0 ? mx[0] : ls[0], tag));
+    }
+  }
+  lds_barrier();
   return true;
 }
 
@@ -2465,6 +2581,10 @@ __global__ __launch_bounds__(ILL_WG_THREADS, 1) void ill_pass_kernel(IllPassArgs
       if (!role_prep<T>(a, H, S.prep1, t)) return;
       lds_barrier();
     }
+  }
+  if constexpr (T == 1) {
+    if (wg >= ILL_R_HELP0 && wg < ILL_R_HELP0 + ILL_HELP_R * ILL_NH)
+      if (!role_help<T>(a, H, S.att, wg - ILL_R_HELP0, ill_stage)) return;
   }
   trace_mark(a, ILL_TR_TAIL);
   if (!role_lmh<T>(a, H, S.lmh, ill_stage)) return;
