@@ -171,6 +171,7 @@ struct ill_engine {
   float* opart = nullptr;   // split-K partials of the layer-by-layer GEMMs; row kernels: attention states
   float* ssq = nullptr;     // [ILL_OP_MAXM][ROW_SSQ] sum-of-squares partials of the row kernels
   int q8g = 64;
+  int oprows = 0;   // rows of a prompt chunk at most: ILL_OP_MAXM, or the context if that is shorter
   hipEvent_t ev0 = nullptr, ev1 = nullptr;   // bracket the last single-pass launch
 };
 
@@ -557,6 +558,7 @@ int ill_create(const char* path, int max_context, int max_pass, int max_steps, i
   e->layers = layers;
   e->vocab = vocab;
   e->maxctx = (max_context + 63) / 64 * 64;
+  e->oprows = std::min(ILL_OP_MAXM, e->maxctx);
   e->maxpass = max_pass;
   e->maxsteps = max_steps;
   auto cleanup = [&](int rc) {
@@ -758,7 +760,7 @@ int ill_create(const char* path, int max_context, int max_pass, int max_steps, i
   const size_t kvb = (size_t)layers * ILL_NKV * e->maxctx * 64 * 2;
   e->acc_bytes = (size_t)2 * layers * ILL_NKIND * 16 * ILL_ACC_ROW * 8;
   bool ok = dalloc((void**)&e->dlayers, sizeof(IllLayerW) * layers) && dalloc((void**)&e->st, 64) && dalloc((void**)&e->ctl, 64) &&
-            dalloc((void**)&e->ptoks, ILL_OP_MAXM * 4) && dalloc((void**)&e->tree, ILL_TR_INTS * 4) &&
+            dalloc((void**)&e->ptoks, e->oprows * 4) && dalloc((void**)&e->tree, ILL_TR_INTS * 4) &&
             dalloc((void**)&e->rope, (size_t)(e->maxctx + 16) * 32 * 8) && dalloc((void**)&e->kc, kvb) && dalloc((void**)&e->vt, kvb) &&
             dalloc((void**)&e->acc, e->acc_bytes) &&
             dalloc((void**)&e->lmp, (size_t)ILL_WG * 16 * 2 * 8) && dalloc((void**)&e->pub, (size_t)ILL_PUB_WORDS * 8) &&
@@ -766,11 +768,11 @@ int ill_create(const char* path, int max_context, int max_pass, int max_steps, i
             dalloc((void**)&e->hs, (size_t)ILL_NH * (e->maxctx / 64) * ILL_HELP_W * 8) &&
             dalloc((void**)&e->logits, (size_t)16 * vocab * 4) &&
             dalloc((void**)&e->out_dev, (size_t)max_steps * 4);
-  ok = ok && dalloc((void**)&e->dolayers, sizeof(OpLayerW) * layers) && dalloc((void**)&e->octx.x, (size_t)ILL_OP_MAXM * ILL_H * 4) &&
-       dalloc((void**)&e->octx.xn, (size_t)ILL_OP_MAXM * ILL_H * 2) && dalloc((void**)&e->octx.q, (size_t)ILL_OP_MAXM * ILL_H * 4) &&
-       dalloc((void**)&e->octx.ao, (size_t)ILL_OP_MAXM * ILL_H * 2) && dalloc((void**)&e->octx.h, (size_t)ILL_OP_MAXM * ILL_FF * 2) &&
+  ok = ok && dalloc((void**)&e->dolayers, sizeof(OpLayerW) * layers) && dalloc((void**)&e->octx.x, (size_t)e->oprows * ILL_H * 4) &&
+       dalloc((void**)&e->octx.xn, (size_t)e->oprows * ILL_H * 2) && dalloc((void**)&e->octx.q, (size_t)e->oprows * ILL_H * 4) &&
+       dalloc((void**)&e->octx.ao, (size_t)e->oprows * ILL_H * 2) && dalloc((void**)&e->octx.h, (size_t)e->oprows * ILL_FF * 2) &&
        dalloc((void**)&e->octx.amax, (size_t)(vocab / OP_BN) * 16 * 8) && dalloc((void**)&e->opart, ILL_OP_PART_BYTES) &&
-       dalloc((void**)&e->ssq, (size_t)ILL_OP_MAXM * ROW_SSQ * 4);
+       dalloc((void**)&e->ssq, (size_t)e->oprows * ROW_SSQ * 4);
   if (!ok) return cleanup(fail(ILL_E_HIP, "device buffer allocation failed"));
   if (hipMemcpy(e->dolayers, e->holayers.data(), sizeof(OpLayerW) * layers, hipMemcpyHostToDevice) != hipSuccess)
     return cleanup(fail(ILL_E_HIP, "layer table upload failed"));
@@ -938,9 +940,9 @@ int ill_prefill(ill_engine* e, const int32_t* toks, int n, int write_logits) {
   // encodePrefill commits through k_commit_spec when speculation is on (Engine.swift:588-601):
   // the State's tspec > 1 makes the prompt's commit draft the first verify pass
   const int fin = s.tspec > 1 ? 2 : 1;
-  if (e->fmt != 2 || n > 16) {   // layer-by-layer path, chunks of up to ILL_OP_MAXM rows
-    for (int c0 = 0; c0 < n; c0 += ILL_OP_MAXM) {
-      const int rows = n - c0 < ILL_OP_MAXM ? n - c0 : ILL_OP_MAXM;
+  if (e->fmt != 2 || n > 16) {   // layer-by-layer path, chunks of up to oprows rows
+    for (int c0 = 0; c0 < n; c0 += e->oprows) {
+      const int rows = n - c0 < e->oprows ? n - c0 : e->oprows;
       const bool last = c0 + rows == n;
       HCK(hipMemcpyAsync(e->ptoks, toks + c0, rows * 4, hipMemcpyHostToDevice, e->stream));
       if ((rc = write_pos_n(e, pos, rows))) return rc;

@@ -25,7 +25,11 @@
 #pragma once
 #include "ill_pass.h"
 
-#define ILL_OP_MAXM 512
+// Rows of a prompt chunk at most (less where the context is shorter). The GEMMs need many rows
+// to fill the chip: whole prompts in chunks of 512 / 1024 / 2048 rows took 16.9 / 13.6 / 11.6 ms
+// (f16, 4000 tokens), 7.6 / 6.0 / 5.0 (2000), 3.2 / 2.3 / 2.3 (700); q4 18.7 / 15.0 / 12.7 (4000).
+// The activations of 4096 rows take 90 MB.
+#define ILL_OP_MAXM 4096
 
 struct OpMat {
   const uint8_t* w;    // q4 nibbles, q8 int8 or f16 halves, tiled (op_wt_off, op_w4_off)
