@@ -368,10 +368,17 @@ void op_head(ill_engine* e, const OpCtx& c, int row0, int n) {
   hipLaunchKernelGGL((op_gemm_ring_kernel<FMT, 16, OP_LMH, ST>), dim3(c.emb.N / OP_BN, 1, 1), dim3(256), 0, e->stream, g);
 }
 
-// Attention over a prompt chunk's 16-row blocks blk0 .. (every query head).
+// Attention over a prompt chunk's 16-row blocks blk0 .. (every query head): chunks shared through
+// LDS from as many blocks on as fill the chip that way, whole prompts in ms, shared / not: q8 and
+// f16 512 rows 1.83 / 1.79, 1000 2.64 / 2.62, 1500 3.62 / 3.68, 4000 7.75 / 8.09; q4 (whose cache
+// rows are slower to read in fragments) 200 1.39 / 1.37, 512 1.81 / 1.89, 4000 7.36 / 11.2.
 template <int FMT>
 void op_attn_rows(ill_engine* e, int layer, int M, int blk0) {
-  hipLaunchKernelGGL(op_attn_rows_kernel<FMT != 2>, dim3((M + 15) / 16 - blk0, ILL_NH), dim3(64 * OP_RW), 0, e->stream, e->octx, layer, M, blk0);
+  const int nb = (M + 15) / 16 - blk0;
+  if (nb >= (FMT == 2 ? 24 : 72))
+    hipLaunchKernelGGL((op_attn_rows_kernel<FMT != 2, true, 2>), dim3(4 * nb), dim3(512), 0, e->stream, e->octx, layer, M, blk0);
+  else
+    hipLaunchKernelGGL((op_attn_rows_kernel<FMT != 2, false, 4>), dim3(nb, ILL_NH), dim3(256), 0, e->stream, e->octx, layer, M, blk0);
 }
 
 // The last layer of a prompt chunk after its QKV product. Only the chunk's last row goes on to

@@ -650,157 +650,261 @@ __device__ __forceinline__ void att_combine(const float* m, const float* l, cons
   oo = acc;
 }
 
-// ---- attention of prefill chunks (more than 16 rows): MFMA flash attention --------------
-// One workgroup of OP_RW waves per (16-row block, query head h): chunk c goes to wave
-// c % OP_RW, which folds its chunks in order, and the waves' states are combined at the end
-// in wave order. Row t < M sits at position pos + t and attends to positions 0 .. pos + t,
-// all in the cache (this chunk's QKV kernel has written its own keys and values). Per
-// 64-position chunk: scores (0.125 q) . k on v_mfma_f32_16x16x32_f16 with q split into f16
-// high and low parts (products as accurate as fp32 q), the causal mask, the row softmax statistics (maximum, sum of exponentials) folded chunk by chunk with
-// the rule of the other attention kernels, and O += P V with P split the same way. A wave's
-// next chunk's keys and values stream in while one is evaluated.
-#define OP_RW 4
-// P round trip through LDS: rows of 68 floats, so that the row-strided writes (4 kg + j)
-// and the per-lane row reads (n) spread over the 64 banks (rows of 64 put a wave's 16 row
-// reads, and its 4 kg groups' writes, on the same banks)
-#define OP_PLD 68
-template <bool SWZ>   // the K/V cache layout (ill_common.h): swizzled for q8 / f16, rows for q4
-__global__ __launch_bounds__(64 * OP_RW) void op_attn_rows_kernel(OpCtx c, int layer, int M, int blk0) {
-  __shared__ __attribute__((aligned(16))) float pbw[OP_RW][16 * OP_PLD];
-  __shared__ float sm_[OP_RW][16], sl_[OP_RW][16], so_[OP_RW][16][64];
+#define OP_ATTN_LAG 8.0f
+// ---- attention of prompt chunks of more than 16 rows: MFMA flash attention ----------------
+// A wave evaluates 16 rows of one query head against 64-position chunks of the cache (this
+// chunk's QKV kernel has written its own keys and values): row t < M sits at position pos + t and
+// attends to positions 0 .. pos + t. Scores are K rows x rows of q and outputs V dims x rows
+// (v_mfma_f32_16x16x32_f16), so the softmax statistics of row n are lane n's, and the keys of an
+// MFMA block are dealt out (block b, row 4 kg + r: key 32 (b / 2) + 8 kg + 4 (b % 2) + r) such
+// that the probabilities a lane holds are the next product's operand as they stand: no pass
+// through LDS, no reduction across the 16 lanes of a row. q and P are split into f16 high and
+// low parts (products as accurate as fp32 q and P). The sums of the exponentials stay per lane
+// until the end, and the value products accumulate onto the output. The next chunk streams in
+// meanwhile. The kernel is bound by the vector instructions per score.
+// GRP: a workgroup per (16 rows, four or three heads of a KV group), SPL waves per head taking turns
+// at the chunks; SPL chunks' keys and values at a time go from memory straight into LDS once for
+// the heads (16 KB each, two buffers: the next ones stream in meanwhile). For few blocks (GRP false): SPL waves per (16 rows, query head), chunk c to wave c % SPL, their states combined in
+// wave order. 2000 rows from position 0: 61 us per layer (q4 79) with scores as rows x keys and P
+// turned through LDS, every head reading K and V itself; 40 (101) with the layout above, 44 (45)
+// with chunks shared through LDS by seven heads, 37 (39) with two waves per head and the lazy
+// maximum, 29 (30) with the heads on two workgroups, so that the causal load evens out.
+template <bool SWZ, bool GRP, int SPL>   // SWZ: the K/V cache layout (ill_common.h): swizzled for q8 / f16, rows for q4
+__global__ __launch_bounds__(64 * SPL * (GRP ? 4 : 1), GRP ? 1 : 2) void op_attn_rows_kernel(OpCtx c, int layer, int M, int blk0) {
   const OpHdr hd = op_hdr(c);
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, kg = lane >> 4, n = lane & 15;
-  float* pb = pbw[w];
-  const int t0 = 16 * (blk0 + (int)blockIdx.x), h = blockIdx.y, g = h / 7;
+  // GRP: 4 workgroups per block, (KV group, its first four or last three heads), in descending
+  // order of the blocks' chunks; the second 256 (a CU's second workgroup) in ascending order
+  int id = blockIdx.x;
+  if (GRP && (id >> 8) == 1) id = min(511, (int)gridDim.x - 1) - (id - 256);
+  const int t0 = 16 * (blk0 + (GRP ? ((int)gridDim.x >> 2) - 1 - (id >> 2) : id));
+  const int hw = GRP ? w & 3 : 0;
+  const int g = GRP ? (id >> 1) & 1 : (int)blockIdx.y / 7, h = GRP ? 7 * g + 4 * (id & 1) + min(hw, 2 + (~id & 1)) : (int)blockIdx.y;
+  const bool live = !GRP || !(id & 1) || hw < 3;   // (the last three heads' fourth wave only loads)
+  const int sp = GRP ? w >> 2 : w;   // this wave's chunks: sp, sp + SPL, ..
+  const int t = min(t0 + n, M - 1);   // (rows past the last repeat it and are not stored)
+  float4 qf[2][2];
+#pragma unroll
+  for (int ks = 0; ks < 2; ks++)
+#pragma unroll
+    for (int i = 0; i < 2; i++) qf[ks][i] = gld((const float4*)(c.q + (size_t)t * ILL_H + h * 64 + 32 * ks + 8 * kg) + i);
+  const uint16_t* kb = c.kc + ((size_t)layer * ILL_NKV + g) * c.maxctx * 64;
+  const uint16_t* vb = c.vt + ((size_t)layer * ILL_NKV + g) * c.maxctx * 64;
+  struct Frag {
+    uint4 k[4][2], v[4][2];
+  };
+  auto fetch = [&](int ch, Frag& f) {
+#pragma unroll
+    for (int b = 0; b < 4; b++)
+#pragma unroll
+      for (int ks = 0; ks < 2; ks++)
+        f.k[b][ks] = gld((const uint4*)(kb + kv_k_off(64 * ch + 32 * (b >> 1) + 8 * (n >> 2) + 4 * (b & 1) + (n & 3), 32 * ks + 8 * kg, SWZ)));
+#pragma unroll
+    for (int nb = 0; nb < 4; nb++)
+#pragma unroll
+      for (int s = 0; s < 2; s++) f.v[nb][s] = gld((const uint4*)(vb + kv_v_off(64 * ch + 32 * s + 8 * kg, 16 * nb + n, SWZ)));
+  };
   const int pos = hd.pos;
-  // A operand: lane (kg, n) holds row t0 + n, dims 32 ks + 8 kg + i
-  v8h qa[2][2];
-  {
-    const float* qr = c.q + (size_t)min(t0 + n, M - 1) * ILL_H + h * 64;
+  const int L = pos + t + 1;
+  const int nch = (pos + min(t0 + 16, M) + 63) >> 6;   // of the block's last row
+  const int full = (pos + t0 + 1) >> 6;                // chunks whole for every row
+  auto over_kg = [](float v, auto op) {   // over the lanes of the same row
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_int(v), __float_as_int(v), false, false);
+    v = op(__int_as_float((int)a[0]), __int_as_float((int)a[1]));
+    const auto q = __builtin_amdgcn_permlane32_swap(__float_as_int(v), __float_as_int(v), false, false);
+    return op(__int_as_float((int)q[0]), __int_as_float((int)q[1]));
+  };
+  v8h qh[2], ql[2];   // q / 8 * log2(e): the scores are exponents of 2
 #pragma unroll
-    for (int ks = 0; ks < 2; ks++) {
-      const uint4 a0 = gld((const uint4*)(qr + 32 * ks + 8 * kg)), a1 = gld((const uint4*)(qr + 32 * ks + 8 * kg + 4));
-      const uint32_t x[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
+  for (int ks = 0; ks < 2; ks++) {
+    const float v[8] = {qf[ks][0].x, qf[ks][0].y, qf[ks][0].z, qf[ks][0].w, qf[ks][1].x, qf[ks][1].y, qf[ks][1].z, qf[ks][1].w};
 #pragma unroll
-      for (int i = 0; i < 8; i++) {
-        const float v = __uint_as_float(x[i]) * 0.125f;
-        const _Float16 hi = (_Float16)v;
-        qa[ks][0][i] = hi;
-        qa[ks][1][i] = (_Float16)(v - (float)hi);
-      }
+    for (int i = 0; i < 8; i++) {
+      const float x = v[i] * (0.125f * 1.4426950408889634f);
+      const _Float16 hi = (_Float16)x;
+      qh[ks][i] = hi;
+      ql[ks][i] = (_Float16)(x - (float)hi);
     }
   }
-  int Lr[4];   // L of this lane's rows t0 + 4 kg + j (0: no row)
+  // The exponents' reference Mx of a row follows its maximum lazily: the score products start from
+  // -Mx, and only when a score comes out above OP_ATTN_LAG is Mx moved up and everything summed so
+  // far rescaled (p <= 2^OP_ATTN_LAG stays far inside f16 and fp32). The first chunk sets it.
+  float Mx = 0.f, Ls = 0.f;   // Ls: this lane's keys only
+  bool first = true;
+  v4f O[4];
 #pragma unroll
-  for (int j = 0; j < 4; j++) Lr[j] = t0 + 4 * kg + j < M ? pos + t0 + 4 * kg + j + 1 : 0;
-  const int nch = (pos + min(t0 + 16, M) + 63) >> 6;
-  const uint16_t* kbase = c.kc + ((size_t)layer * ILL_NKV + g) * c.maxctx * 64;
-  const uint16_t* vbase = c.vt + ((size_t)layer * ILL_NKV + g) * (c.maxctx / 64) * 64 * 64;
-  float Mx[4], Ls[4], O[4][4];
-#pragma unroll
-  for (int j = 0; j < 4; j++) {
-    Mx[j] = -INFINITY;
-    Ls[j] = 0.f;
-#pragma unroll
-    for (int nb = 0; nb < 4; nb++) O[nb][j] = 0.f;
-  }
-  KVFrag f;
-  if (w < nch) kv_fetch<SWZ>(kbase, vbase, w, lane, f);
-  for (int ch = w; ch < nch; ch += OP_RW) {
-    KVFrag fn;
-    const bool more = ch + OP_RW < nch;
-    if (more) kv_fetch<SWZ>(kbase, vbase, ch + OP_RW, lane, fn);
-    float sc[4][4];
+  for (int nb = 0; nb < 4; nb++) O[nb] = (v4f){0.f, 0.f, 0.f, 0.f};
+  auto eval = [&](int ch, const Frag& f) {
+    v4f sc[4];
 #pragma unroll
     for (int b = 0; b < 4; b++) {
-      v4f sv = {0.f, 0.f, 0.f, 0.f};
-      sv = __builtin_amdgcn_mfma_f32_16x16x32_f16(qa[0][0], u4_to_v8h(f.k[b][0]), sv, 0, 0, 0);
-      sv = __builtin_amdgcn_mfma_f32_16x16x32_f16(qa[0][1], u4_to_v8h(f.k[b][0]), sv, 0, 0, 0);
-      sv = __builtin_amdgcn_mfma_f32_16x16x32_f16(qa[1][0], u4_to_v8h(f.k[b][1]), sv, 0, 0, 0);
-      sv = __builtin_amdgcn_mfma_f32_16x16x32_f16(qa[1][1], u4_to_v8h(f.k[b][1]), sv, 0, 0, 0);
-      const int vp = 64 * ch + 16 * b + n;
+      v4f d = {-Mx, -Mx, -Mx, -Mx};
 #pragma unroll
-      for (int j = 0; j < 4; j++) sc[b][j] = vp < Lr[j] ? sv[j] : -INFINITY;
-    }
-    float mx[4], ls[4];
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      mx[j] = gmax<16>(fmaxf(fmaxf(sc[0][j], sc[1][j]), fmaxf(sc[2][j], sc[3][j])));
-      const float ms = mx[j] == -INFINITY ? 0.f : mx[j];   // a row with no position here: p = 0
-      float sum = 0.f;
-#pragma unroll
-      for (int b = 0; b < 4; b++) {
-        sc[b][j] = att_exp(sc[b][j] - ms);
-        sum += sc[b][j];
+      for (int ks = 0; ks < 2; ks++) {
+        d = __builtin_amdgcn_mfma_f32_16x16x32_f16(u4_to_v8h(f.k[b][ks]), qh[ks], d, 0, 0, 0);
+        d = __builtin_amdgcn_mfma_f32_16x16x32_f16(u4_to_v8h(f.k[b][ks]), ql[ks], d, 0, 0, 0);
       }
-      ls[j] = gsum<16>(sum);
-#pragma unroll
-      for (int b = 0; b < 4; b++) pb[(4 * kg + j) * OP_PLD + 16 * b + n] = sc[b][j];
+      sc[b] = d;
     }
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    if (ch >= full) {   // (wave-uniform) positions past a row
+#pragma unroll
+      for (int b = 0; b < 4; b++)
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+          if (64 * ch + 32 * (b >> 1) + 8 * kg + 4 * (b & 1) + r >= L) sc[b][r] = -INFINITY;
+    }
+    float mc = sc[0][0];
+#pragma unroll
+    for (int b = 0; b < 4; b++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) mc = fmaxf(mc, sc[b][r]);
+    if (first || __any(mc > OP_ATTN_LAG)) {   // (wave-uniform)
+      mc = over_kg(mc, OpMaxF{});
+      // up by the excess; the first chunk: to the maximum (a row with no position in it stays at 0)
+      const float up = first ? (mc == -INFINITY ? 0.f : mc) : fmaxf(mc, 0.f);
+      const float sa = __builtin_amdgcn_exp2f(-up);
+      first = false;
+      Mx += up;
+      Ls *= sa;
+#pragma unroll
+      for (int nb = 0; nb < 4; nb++) O[nb] *= sa;
+#pragma unroll
+      for (int b = 0; b < 4; b++) sc[b] -= up;
+    }
     v8h ph[2], pl[2];
 #pragma unroll
-    for (int ks = 0; ks < 2; ks++) {
+    for (int b = 0; b < 4; b++)
 #pragma unroll
-      for (int i = 0; i < 8; i++) {
-        const float p = pb[n * OP_PLD + 32 * ks + 8 * kg + i];
-        const _Float16 hi = (_Float16)p;
-        ph[ks][i] = hi;
-        pl[ks][i] = (_Float16)(p - (float)hi);
+      for (int r = 0; r < 4; r += 2) {
+        const float p0 = __builtin_amdgcn_exp2f(sc[b][r]), p1 = __builtin_amdgcn_exp2f(sc[b][r + 1]);
+        Ls += p0;
+        Ls += p1;
+        const _Float16 h0 = (_Float16)p0, h1 = (_Float16)p1;
+        ph[b >> 1][4 * (b & 1) + r] = h0;
+        ph[b >> 1][4 * (b & 1) + r + 1] = h1;
+        pl[b >> 1][4 * (b & 1) + r] = (_Float16)fmaf((float)h0, -1.f, p0);
+        pl[b >> 1][4 * (b & 1) + r + 1] = (_Float16)fmaf((float)h1, -1.f, p1);
       }
+#pragma unroll
+    for (int nb = 0; nb < 4; nb++)
+#pragma unroll
+      for (int s = 0; s < 2; s++) {
+        O[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(u4_to_v8h(f.v[nb][s]), ph[s], O[nb], 0, 0, 0);
+        O[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(u4_to_v8h(f.v[nb][s]), pl[s], O[nb], 0, 0, 0);
+      }
+  };
+  __shared__ __attribute__((aligned(16))) uint4 kv[GRP ? 2 : 1][GRP ? SPL * 1024 : 1];
+  if constexpr (GRP) {
+    // 16-byte units of the chunk as stored (K 0 .. 511, V 512 .. 1023), except that the rows layout's
+    // 8 units per key or dim are permuted among themselves, so that the eight lanes that LDS
+    // serves at once (fragment reads: keys 0-3 and 8-11, or eight dims) fall on different banks
+    auto kswz = [](int key) { return SWZ ? 0 : (key & 3) | ((key >> 1) & 4); };
+    auto load = [&](int it, int buf) {   // (chunks past the last repeat it)
+      for (int i = w; i < 16 * SPL; i += 4 * SPL) {
+        const int u = 64 * (i & 7) + lane, ch = min(SPL * it + (i >> 4), nch - 1);
+        const bool k = (i & 15) < 8;
+        const int src = SWZ ? u : (u & ~7) | ((u & 7) ^ (k ? kswz(u >> 3) : (u >> 3) & 7));
+        op_lds_dma16((const uint4*)((k ? kb : vb) + (size_t)4096 * ch) + src, &kv[buf][64 * i]);
+      }
+    };
+    load(0, 0);
+    for (int it = 0; SPL * it < nch; it++) {
+      op_vm_barrier<0>();   // these chunks are in LDS, and every wave is done with the buffer filled next
+      if (SPL * (it + 1) < nch) load(it + 1, (it + 1) & 1);
+      const int ch = SPL * it + sp;
+      if (ch >= nch || !live) continue;   // (ch: the last turn)
+      Frag f;
+      const uint4* b0 = kv[it & 1] + 1024 * sp;
+#pragma unroll
+      for (int b = 0; b < 4; b++)
+#pragma unroll
+        for (int ks = 0; ks < 2; ks++) {
+          const int key = 32 * (b >> 1) + 8 * (n >> 2) + 4 * (b & 1) + (n & 3), dg = 4 * ks + kg;
+          f.k[b][ks] = b0[SWZ ? dg * 64 + key : key * 8 + (dg ^ kswz(key))];
+        }
+#pragma unroll
+      for (int nb = 0; nb < 4; nb++)
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+          const int dim = 16 * nb + n, pg = 4 * s + kg;
+          f.v[nb][s] = b0[512 + (SWZ ? pg * 64 + dim : dim * 8 + (pg ^ (dim & 7)))];
+        }
+      eval(ch, f);
     }
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  } else if (sp < nch) {
+    const int c0 = sp;
+    Frag f0, f1;
+    fetch(c0, f0);
+    for (int ch = c0;; ch += 2 * SPL) {   // two chunks per turn: the buffers swap without copies
+      // (past the last chunk the fetch repeats it, so the loads in flight never depend on a branch)
+      fetch(min(ch + SPL, nch - 1), f1);
+      __builtin_amdgcn_sched_barrier(0);
+      eval(ch, f0);
+      if (ch + SPL >= nch) break;
+      fetch(min(ch + 2 * SPL, nch - 1), f0);
+      __builtin_amdgcn_sched_barrier(0);
+      eval(ch + SPL, f1);
+      if (ch + 2 * SPL >= nch) break;
+    }
+  }
+  Ls = over_kg(Ls, OpAddF{});
+  if (Ls == 0.f) Mx = -INFINITY;   // a row with no position in this wave's chunks
+  if constexpr (GRP) {
+    static_assert(SPL == 1 || SPL == 2, "states of two waves per head");
+    if constexpr (SPL == 2) {   // the two waves' states, in LDS over the chunks
+      float* st = (float*)kv + hw * 18 * 64;
+      lds_barrier();
+      if (sp == 1) {
+        st[lane] = Mx;
+        st[64 + lane] = Ls;
+#pragma unroll
+        for (int nb = 0; nb < 4; nb++) *(v4f*)&st[128 + 256 * nb + 4 * lane] = O[nb];
+      }
+      lds_barrier();
+      if (sp == 1) return;
+      const float m1 = st[lane], mm = fmaxf(Mx, m1);
+      const float e0 = __builtin_amdgcn_exp2f(Mx - mm), e1 = __builtin_amdgcn_exp2f(m1 - mm);
+      Ls = Ls * e0 + st[64 + lane] * e1;
+#pragma unroll
+      for (int nb = 0; nb < 4; nb++) O[nb] = O[nb] * e0 + *(const v4f*)&st[128 + 256 * nb + 4 * lane] * e1;
+    }
+    if (hd.done || !live || t0 + n >= M) return;
+    const float inv = 1.0f / Ls;
 #pragma unroll
     for (int nb = 0; nb < 4; nb++) {
-      v4f acc = {0.f, 0.f, 0.f, 0.f};
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ph[0], u4_to_v8h(f.v[nb][0]), acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(pl[0], u4_to_v8h(f.v[nb][0]), acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ph[1], u4_to_v8h(f.v[nb][1]), acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(pl[1], u4_to_v8h(f.v[nb][1]), acc, 0, 0, 0);
+      uint2 y;
+      y.x = f2h(O[nb][0] * inv) | (f2h(O[nb][1] * inv) << 16);
+      y.y = f2h(O[nb][2] * inv) | (f2h(O[nb][3] * inv) << 16);
+      gst((gu32x2*)(c.ao + (size_t)t * ILL_H + h * 64 + 16 * nb + 4 * kg), (gu32x2){y.x, y.y});
+    }
+  } else {
+    __shared__ float sm_[SPL][16], sl_[SPL][16];
+    __shared__ __attribute__((aligned(16))) float so_[SPL][16][68];
+    if (kg == 0) {
+      sm_[w][n] = Mx;
+      sl_[w][n] = Ls;
+    }
 #pragma unroll
-      for (int j = 0; j < 4; j++) {
-        if (mx[j] == -INFINITY) continue;   // nothing of this row in the chunk
-        const AttScale k = att_scale(Mx[j], mx[j]);
-        O[nb][j] = att_fold(O[nb][j], acc[j], k);
-        if (nb == 3) {
-          Ls[j] = att_fold(Ls[j], ls[j], k);
-          Mx[j] = k.mn;
-        }
+    for (int nb = 0; nb < 4; nb++) *(v4f*)&so_[w][n][16 * nb + 4 * kg] = O[nb];
+    __syncthreads();
+    if (hd.done) return;
+    for (int i = threadIdx.x; i < 16 * 16; i += 64 * SPL) {   // row i / 16, dims 4 (i % 16) ..
+      const int r = i >> 4, d = 4 * (i & 15);
+      if (t0 + r >= M) break;
+      float mm = sm_[0][r];
+#pragma unroll
+      for (int k = 1; k < SPL; k++) mm = fmaxf(mm, sm_[k][r]);
+      float l = 0.f;
+      v4f o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k = 0; k < SPL; k++) {
+        const float e = __builtin_amdgcn_exp2f(sm_[k][r] - mm);
+        l += sl_[k][r] * e;
+        o += *(const v4f*)&so_[k][r][d] * e;
       }
+      gst((gu32x2*)(c.ao + (size_t)(t0 + r) * ILL_H + h * 64 + d),
+          (gu32x2){f2h(o[0] / l) | (f2h(o[1] / l) << 16), f2h(o[2] / l) | (f2h(o[3] / l) << 16)});
     }
-    if (more) f = fn;
-  }
-  // the waves' states, combined in wave order against their maximum
-#pragma unroll
-  for (int j = 0; j < 4; j++) {
-    if (n == 0) {
-      sm_[w][4 * kg + j] = Mx[j];
-      sl_[w][4 * kg + j] = Ls[j];
-    }
-#pragma unroll
-    for (int nb = 0; nb < 4; nb++) so_[w][4 * kg + j][16 * nb + n] = O[nb][j];
-  }
-  __syncthreads();
-  if (hd.done) return;
-  const int r = threadIdx.x >> 4, t = t0 + r;
-  if (t >= M) return;
-  float m[OP_RW], l[OP_RW];
-#pragma unroll
-  for (int i = 0; i < OP_RW; i++) {
-    m[i] = sm_[i][r];
-    l[i] = sl_[i][r];
-  }
-#pragma unroll
-  for (int q = 0; q < 4; q++) {
-    const int d = (threadIdx.x & 15) + 16 * q;
-    float o[OP_RW];
-#pragma unroll
-    for (int i = 0; i < OP_RW; i++) o[i] = so_[i][r][d];
-    float mo, lo, oo;
-    att_combine<OP_RW>(m, l, o, mo, lo, oo);
-    gst((uint16_t*)(c.ao + (size_t)t * ILL_H + h * 64 + d), (uint16_t)__half_as_ushort(__float2half(oo / lo)));
   }
 }
 

@@ -106,3 +106,30 @@ def test_prompts_at_the_row_kernels_edges(fmt, tmp_path):
             assert metrics.rel_l2(e.read_logits(0), ref) <= REL_L2_TOL, parts
     finally:
         e.close()
+
+
+@pytest.mark.parametrize("fmt", [F.FMT_Q4, F.FMT_F16], ids=["q4", "f16"])
+def test_prompt_attention_shapes(fmt, tmp_path):
+    """Both shapes of the prompt attention (chunks shared through LDS, waves per head) at the block
+    counts around the switch (24 blocks of 16 rows for q4, 72 for f16), odd and even chunk counts
+    and last blocks, and second calls that start inside a 64-position chunk: last-row logits
+    against the oracle."""
+    from instantllm_amd.engine import Engine
+    path = str(tmp_path / "m.ill")
+    synth.build_model(path, fmt, seed=6, shape=synth.ModelShape(layers=2, vocab=VOCAB))
+    m = qwen.Model(illread.load(path))
+    e = Engine(path, max_context=2176, max_pass=16, max_steps=64)
+    toks = [int(t) for t in np.random.default_rng(710 + fmt).integers(0, VOCAB, size=2100)]
+    cuts = ((368,), (369,), (385,), (700,), (40, 1152), (77, 1130), (1300, 750)) if fmt == F.FMT_Q4 else \
+           ((1136,), (1137,), (1153,), (40, 1152), (77, 1130), (1300, 750))
+    try:
+        for parts in cuts:
+            e.set_state(pos=0, n=1, maxsteps=64, eos=NO_EOS)
+            n = 0
+            for k in parts:
+                e.prefill(toks[n:n + k], write_logits=True)
+                n += k
+            ref = m.forward(toks[:n], m.new_cache(n + 1))
+            assert metrics.rel_l2(e.read_logits(0), ref) <= REL_L2_TOL, parts
+    finally:
+        e.close()
