@@ -762,7 +762,8 @@ __global__ __launch_bounds__(64 * SPL * (GRP ? 4 : 1), GRP ? 1 : 2) void op_attn
       mc = over_kg(mc, OpMaxF{});
       // up by the excess; the first chunk: to the maximum (a row with no position in it stays at 0)
       const float up = first ? (mc == -INFINITY ? 0.f : mc) : fmaxf(mc, 0.f);
-      const float sa = __builtin_amdgcn_exp2f(-up);
+      // (nothing is summed before the first chunk, whose maximum may be far below 0: 0 * 2^-up would be NaN)
+      const float sa = first ? 1.f : __builtin_amdgcn_exp2f(-up);
       first = false;
       Mx += up;
       Ls *= sa;
