@@ -315,7 +315,7 @@ int write_pos_n(ill_engine* e, int pos, int n) {
 }
 
 // ---- layer-by-layer path -----------------------------------------------------------------
-#define ILL_OP_PART_BYTES (16u << 20)   // >= slices x rows x N x 4 of every split GEMM
+#define ILL_OP_PART_BYTES (32u << 20)   // >= slices x rows x N x 4 of every split GEMM
 
 OpGemmArgs op_args(ill_engine* e, const __half* A, const OpMat& W, int M, int layer) {
   OpGemmArgs g{};
@@ -343,19 +343,24 @@ bool op_gemm(ill_engine* e, const __half* A, const OpMat& W, int M, int layer, c
     // kernel): 512 rows, f16, 13.9 us against 9.7 + 5.4 us split three ways
     hipLaunchKernelGGL((op_gemm_ring_kernel<FMT, 32, EPI, OP_RING_ST(FMT, EPI)>), dim3(ntn, (M + 31) / 32, 1), dim3(256), 0, e->stream, g);
     return false;
+  } else {
+    const int mt = (M + 63) / 64;
+    int S = 1;
+    if constexpr (EPI == OP_RESID) {
+      // K slices: as many as put about one tile on every CU; three where that puts up to two
+      // tiles on every CU (129-170 tiles; 1500 rows: whole prompts 3.30 -> 2.94 ms
+      // q4, 3.45 -> 3.03 q8, 3.26 -> 3.00 f16; at 2000 and 3000 rows splitting gained nothing)
+      const int tiles = ntn * mt, cap = (int)(ILL_OP_PART_BYTES / ((size_t)M * W.N * 4));   // partial buffer
+      S = tiles > 128 && 3 * tiles <= 512 ? 3 : std::max(1, 256 / tiles);
+      S = std::max(1, std::min(std::min(S, nsteps / 4), std::min(OP_MAXS, cap)));
+      g.ksteps = (nsteps + S - 1) / S;
+      S = (nsteps + g.ksteps - 1) / g.ksteps;
+    }
+    hipLaunchKernelGGL((op_gemm_ring_kernel<FMT, 64, EPI, OP_RING_ST(FMT, EPI)>), dim3(ntn, mt, S), dim3(256), 0, e->stream, g);
+    if (S == 1) return false;
+    hipLaunchKernelGGL(op_epi_norm_kernel, dim3(M), dim3(ILL_H), 0, e->stream, g, S, norm_gamma, 0);
+    return true;
   }
-  const int mt = (M + 63) / 64;
-  int S = 1;
-  if constexpr (EPI == OP_RESID) {
-    const int cap = (int)(ILL_OP_PART_BYTES / ((size_t)M * W.N * 4));   // partial buffer
-    S = std::max(1, std::min(std::min(std::min(256 / (ntn * mt), nsteps / 4), OP_MAXS), cap));
-    g.ksteps = (nsteps + S - 1) / S;
-    S = (nsteps + g.ksteps - 1) / g.ksteps;
-  }
-  hipLaunchKernelGGL((op_gemm_ring_kernel<FMT, 64, EPI, OP_RING_ST(FMT, EPI)>), dim3(ntn, mt, S), dim3(256), 0, e->stream, g);
-  if (S == 1) return false;
-  hipLaunchKernelGGL(op_epi_norm_kernel, dim3(M), dim3(ILL_H), 0, e->stream, g, S, norm_gamma, 0);
-  return true;
 }
 
 // The final norm of rows row0 .. row0 + n - 1 (n <= 16) of c.x, the lm_head and its argmax tiles.

@@ -1,10 +1,9 @@
 // Layer-by-layer ("op") path: one kernel per operation, for any number of rows M.
 //
-// It serves what the persistent q4 pass kernel does not:
-// * the prompt prefill in chunks of up to ILL_OP_MAXM rows, where the projections are real
-//   GEMMs (M = 512 -> MFMA-bound), and
-// * every pass of q8 and f16 models (decode steps, verify passes, prefill), whose per-layer
-//   weights do not fit the persistent kernel's LDS stages.
+// It serves what the persistent q4 pass kernel does not: the prompt prefill, in chunks of up to
+// ILL_OP_MAXM rows, and every pass of q8 and f16 models. Up to ROW_MAXM rows run on the row
+// kernels (ill_rows.h); longer chunks on the kernels here: GEMMs streamed through an LDS ring,
+// MFMA flash attention, and the residual with the next RMSNorm.
 //
 // It follows the reference's own encoding (Engine.swift:370-403 encodePrefillLayer2 on
 // gemm3_core, Shaders.swift:1911-2054; the 1-row kernels :1199-1364): per layer
@@ -14,11 +13,10 @@
 // logits, and the commit.
 //
 // Arithmetic: activations in f16 (the reference's G3 path keeps fp16 activations too),
-// weights dequantized to f16 in LDS (q4: s*q + m; q8: s*q; f16: as stored),
+// weights dequantized to f16 (q4: s*q + m; q8: s*q; f16: as stored),
 // v_mfma_f32_16x16x32_f16 with fp32 accumulation over K in a fixed order, fp32 residual
-// stream. Every row's arithmetic is independent of M and of the rows beside it, so a row
-// decoded alone and the same row inside a 16-row pass produce identical bits (the kernels
-// are the same for M = 1 and M = 16; the 64-row tile is used only for prefill chunks).
+// stream. A row's arithmetic does not depend on the rows beside it; passes of up to 16 rows all
+// run on the row kernels, so a row decoded alone and inside a 16-row pass give identical bits.
 //
 // Every kernel reads the position and the stop flag from the device State, so a decode
 // step recorded in a hipGraph replays correctly.
@@ -206,6 +204,7 @@ struct OpGemmArgs {
 };
 
 #define OP_BN 128
+#define OP_HLD 72    // LDS row stride (halves) of a gate/up tile's hidden units
 #define OP_BK 64
 #define OP_MAXS 24   // K slices of a split GEMM at most
 
@@ -273,8 +272,12 @@ __device__ __forceinline__ void epi_qkv(const OpCtx& c, const OpHdr& hd, int lay
   }
 }
 // gate/up rows in groups of 4: g[2q], g[2q+1], u[2q], u[2q+1] (Convert.swift:134-136)
+// SiLU(g) * u on the hardware exp2 and reciprocal (one ulp each in fp32, then f16)
+__device__ __forceinline__ __half silu_mul(float g, float u) {
+  return __float2half(g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * -1.4426950408889634f)) * u);
+}
 __device__ __forceinline__ void epi_silu(const OpCtx& c, int m, int unit, float g, float u) {
-  c.h[(size_t)m * ILL_FF + unit] = __float2half(g / (1.0f + expf(-g)) * u);
+  c.h[(size_t)m * ILL_FF + unit] = silu_mul(g, u);
 }
 
 // Epilogue of a 128-column tile (lane (kg, n) of wave w holds rows m0 + 16 i + 4 kg + r,
@@ -285,12 +288,13 @@ __device__ __forceinline__ void epi_silu(const OpCtx& c, int m, int unit, float 
 template <int BM, int EPI>
 __device__ __forceinline__ void op_gemm_epilogue(const OpGemmArgs& a, const OpHdr& hd, const v4f (&acc)[BM / 16][2], int m0,
                                                  int n0, int kz, int w, int kg, int n, uint64_t (&red)[4][16],
-                                                 int cs_base = -1, const float2* cs = nullptr, const float* qbias = nullptr) {
+                                                 int cs_base = -1, const float2* cs = nullptr, const float* qbias = nullptr,
+                                                 uint16_t* hst = nullptr) {
   constexpr int TM = BM / 16;
   if (hd.done) return;
   const OpCtx& c = a.c;
   const int tid = threadIdx.x;
-  if (gridDim.z > 1) {   // split K: partials for op_epi_kernel
+  if (gridDim.z > 1) {   // split K: partials for op_epi_norm_kernel
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
@@ -328,10 +332,18 @@ __device__ __forceinline__ void op_gemm_epilogue(const OpGemmArgs& a, const OpHd
         for (int h = 0; h < 2; h++) {
           const float mine = acc[i][j][lo ? h : 2 + h], send = acc[i][j][lo ? 2 + h : h];
           const float got = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(send), 0x4e, 0xf, 0xf, false));
-          const int m = m0 + 16 * i + 4 * kg + (lo ? h : 2 + h);
-          if (m < a.M) epi_silu(c, m, (col >> 2) * 2 + u, lo ? mine : got, lo ? got : mine);
+          // into the tile's f16 image in LDS (64 units a row), then stored 16 bytes per lane
+          // (2-byte stores from here, with expf and a division: 70 us at 2000 rows, f16, against 66)
+          hst[(16 * i + 4 * kg + (lo ? h : 2 + h)) * OP_HLD + ((col - n0) >> 2) * 2 + u] =
+              __half_as_ushort(silu_mul(lo ? mine : got, lo ? got : mine));
         }
       }
+    lds_barrier();
+#pragma unroll
+    for (int q = 0; q < BM / 32; q++) {
+      const int r = 32 * q + (tid >> 3), e = 8 * (tid & 7);
+      if (m0 + r < a.M) gst((gu32x4*)(c.h + (size_t)(m0 + r) * ILL_FF + n0 / 2 + e), *(const gu32x4*)(hst + r * OP_HLD + e));
+    }
   } else if constexpr (EPI == OP_QKV) {
     const int b = (n0 + 32 * w) >> 5;
 #pragma unroll
@@ -393,23 +405,22 @@ __device__ __forceinline__ OpTile op_tile_xcd() {
   return {sl % nx, y, sl / nx};
 }
 
-// ---- prefill GEMM, q8 / f16: operands streamed from memory into an LDS ring --------------
-// op_gemm_kernel stages the next k-step (64 columns) in registers, one step ahead (DEPTH 1)
-// or a ring of DEPTH steps, and stores it to LDS. Here the operands go from memory straight
-// into LDS (global_load_lds_dwordx4: lane i of a wave's load writes 16 bytes at the
-// instruction's LDS address + 16 i), into a ring of ST stages, so that ST - 1 k-steps are in
+// ---- prompt GEMM and lm_head: operands streamed from memory into an LDS ring ----------------
+// The operands go from memory straight into LDS (global_load_lds_dwordx4: lane i of a wave's
+// load writes 16 bytes at the instruction's LDS address + 16 i), into a ring of ST stages, so
+// that ST - 1 k-steps (64 columns) are in
 // flight with no registers or LDS stores spent on them. (Per workgroup at 512 rows: 0.7 us
 // to issue the prologue, then 0.3-0.7 us per k-step; the gate/up GEMM, three workgroups per
 // CU, is bound by the LDS traffic of its k-steps: 24 KB written and 48 KB read, the four
 // waves reading the same A rows.) A stage holds
-//   A: BM rows x 64 halves in 16-byte units ordered (row / 16, k / 8, row % 16), so that the
-//      16 lanes of an MFMA operand read 256 contiguous bytes (no bank conflicts);
-//   B: the k-step's block of the tiled weights (128 rows x 64 columns at op_wt_off, 8 KB q8,
-//      16 KB f16) as stored: its units are already in that order;
+//   A: BM rows x 64 halves, row by row, the 8 16-byte units of a row permuted (k / 8 at place
+//      k / 8 ^ row / 2 % 8): eight lanes of a load take a row's whole 128-byte line, and the 16 lanes
+//      of an operand read (16 rows) fall on different banks. (Units ordered (row / 16, k / 8,
+//      row % 16) read without conflicts too, but the loads gathered 16 bytes of 16 rows: AOLD);
+//   B: the k-step's block of the tiled weights (128 rows x 64 columns at op_wt_off, 4 KB q4,
+//      8 KB q8, 16 KB f16) as stored: its units are already in that order;
 //   q8: the block's scales (128 rows x 64 / qg f16, op_st_off), 256 or 512 bytes.
-// q8 weights are dequantized as they leave LDS, with op_store_w's arithmetic, and every
-// output sums the same products in the same order as op_gemm_kernel: the results are
-// identical. The loads are issued in inline assembly: the compiler's own tracking of LDS
+// q8 and q4 weights are dequantized as they leave LDS. The loads are issued in inline assembly: the compiler's own tracking of LDS
 // loads in flight made it wait for all of them before some of the stage's LDS reads (it
 // could not tell the stages apart), which serialized the ring. The wait for the stage about
 // to be read is explicit: vmcnt counts this wave's own loads, and the barrier after it covers
@@ -432,7 +443,8 @@ __device__ __forceinline__ void op_lds_dma4(const void* g, const void* lds) {
 // slower (512-row prefill 1.96 / 2.24 ms against 1.93 / 2.12 ms; 2.17 / 2.55 ms): issuing the
 // longer prologue took 2 us instead of 0.7 and the k-steps were hardly faster. The gate/up
 // GEMM (608 workgroups at 512 rows) takes 2 (f16) / 3 (q8) stages, so that three workgroups
-// fit per CU and all of them run in one round (f16: 1.90 -> 1.86 ms).
+// fit per CU and all of them run in one round (f16: 1.90 -> 1.86 ms); its launch bounds keep the
+// registers to three workgroups too (q8 at 176 registers: 65 us at 2000 rows, at 157: 54).
 #define OP_RING_ST(FMT, EPI) ((EPI) == OP_SILU ? ((FMT) == 0 ? 2 : 3) : ((FMT) == 0 ? 3 : 4))
 template <int FMT, int BM>
 struct OpRing {                                  // sizes in 16-byte units
@@ -454,8 +466,8 @@ __device__ __forceinline__ void op_ring_load(const OpGemmArgs& a, int m0, int n0
     // unit p (BM 16: 128 units, which waves 2, 3 load again into the same bytes, so that every
     // wave issues the same loads)
     const int p = (256 * u + tid) & (R::A - 1);
-    const int row = min(m0 + ((p >> 7) << 4) + (p & 15), a.M - 1);
-    op_lds_dma16(a.A + (size_t)row * K + k0 + 8 * ((p >> 4) & 7), st + ((256 * u + wb) & (R::A - 1)));
+    const int row = min(m0 + (p >> 3), a.M - 1);
+    op_lds_dma16(a.A + (size_t)row * K + k0 + 8 * ((p ^ (p >> 4)) & 7), st + ((256 * u + wb) & (R::A - 1)));
   }
   const uint4* blk = (const uint4*)(a.W.w + (FMT == 2 ? op_w4_off(n0, k0, K) : op_wt_off(n0, k0, K, FMT == 0 ? 2 : 1)));
 #pragma unroll
@@ -468,39 +480,46 @@ __device__ __forceinline__ void op_ring_load(const OpGemmArgs& a, int m0, int n0
   }
 }
 
+// The A operand of half ks of the k-step in stage st: rows 16 i + n.
+__device__ __forceinline__ v8h op_ring_a(const uint4* st, int i, int ks, int kg, int n) {
+  return u4_to_v8h(st[(16 * i + n) * 8 + ((4 * ks + kg) ^ (n >> 1))]);
+}
+// The B operand of half ks of the k-step in stage st: 16-row sub-tile c16 of the weight block.
+template <int FMT, int BM>
+__device__ __forceinline__ v8h op_ring_b(const uint4* st, int c16, int ks, int kg, int n, int qg) {
+  using R = OpRing<FMT, BM>;
+  if constexpr (FMT == 0) {
+    return u4_to_v8h(st[R::A + c16 * 128 + ((kg & 1) * 4 + 2 * ks + (kg >> 1)) * 16 + n]);
+  } else {
+    v8h v;
+    _Float16 o[8];
+    if constexpr (FMT == 2) {
+      const uint32_t x = ((const uint32_t*)(st + R::A + c16 * 32))[((2 * ks + (kg >> 1)) * 16 + n) * 2 + (kg & 1)];
+      const uint32_t sm = ((const uint32_t*)(st + R::A + R::B))[16 * c16 + n];
+      op_q4x8(x, (_Float16)h2f(sm & 0xffff), (_Float16)h2f(sm >> 16), o);
+    } else {
+      const uint2 q = ((const uint2*)(st + R::A + c16 * 64 + (2 * ks + (kg >> 1)) * 16 + n))[kg & 1];
+      const uint16_t* sc = (const uint16_t*)(st + R::A + R::B);
+      const _Float16 s = (_Float16)h2f(sc[(16 * c16 + n) * (64 / qg) + (qg == 32 ? ks : 0)]);
+      op_q8x4(q.x, s, o);
+      op_q8x4(q.y, s, o + 4);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; i++) v[i] = o[i];
+    return v;
+  }
+}
 // The k-step in stage st: lane (kg, n) of wave w, rows 16 i + n, columns 32 w + 16 j + n.
 template <int FMT, int BM>
 __device__ __forceinline__ void op_ring_mma(const uint4* st, int w, int kg, int n, int qg, v4f (&acc)[BM / 16][2]) {
-  using R = OpRing<FMT, BM>;
 #pragma unroll
   for (int ks = 0; ks < 2; ks++) {
     v8h bf[2];
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
-      const int c16 = 2 * w + j;   // 16-row sub-tile of the weight block
-      if constexpr (FMT == 0) {
-        bf[j] = u4_to_v8h(st[R::A + c16 * 128 + ((kg & 1) * 4 + 2 * ks + (kg >> 1)) * 16 + n]);
-      } else if constexpr (FMT == 2) {
-        const uint32_t x = ((const uint32_t*)(st + R::A + c16 * 32))[((2 * ks + (kg >> 1)) * 16 + n) * 2 + (kg & 1)];
-        const uint32_t sm = ((const uint32_t*)(st + R::A + R::B))[16 * c16 + n];
-        _Float16 o[8];
-        op_q4x8(x, (_Float16)h2f(sm & 0xffff), (_Float16)h2f(sm >> 16), o);
-#pragma unroll
-        for (int i = 0; i < 8; i++) bf[j][i] = o[i];
-      } else {
-        const uint2 q = ((const uint2*)(st + R::A + c16 * 64 + (2 * ks + (kg >> 1)) * 16 + n))[kg & 1];
-        const uint16_t* sc = (const uint16_t*)(st + R::A + R::B);
-        const _Float16 s = (_Float16)h2f(sc[(16 * c16 + n) * (64 / qg) + (qg == 32 ? ks : 0)]);
-        _Float16 o[8];
-        op_q8x4(q.x, s, o);
-        op_q8x4(q.y, s, o + 4);
-#pragma unroll
-        for (int i = 0; i < 8; i++) bf[j][i] = o[i];
-      }
-    }
+    for (int j = 0; j < 2; j++) bf[j] = op_ring_b<FMT, BM>(st, 2 * w + j, ks, kg, n, qg);
 #pragma unroll
     for (int i = 0; i < BM / 16; i++) {
-      const v8h af = u4_to_v8h(st[i * 128 + (4 * ks + kg) * 16 + n]);
+      const v8h af = op_ring_a(st, i, ks, kg, n);
 #pragma unroll
       for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af, bf[j], acc[i][j], 0, 0, 0);
     }
@@ -527,10 +546,10 @@ __device__ __forceinline__ void op_ring_wait(int later) {
   }
 }
 
-// Grid, tiles and epilogues as op_gemm_kernel (4 waves; wave w owns columns 32 w .. + 31 of
+// Grid: column tiles x row tiles x K slices (4 waves; wave w owns columns 32 w .. + 31 of
 // the 128-column tile and all BM rows).
 template <int FMT, int BM, int EPI, int ST>
-__global__ __launch_bounds__(256) void op_gemm_ring_kernel(OpGemmArgs a) {
+__global__ __launch_bounds__(256, EPI == OP_SILU ? 3 : 2) void op_gemm_ring_kernel(OpGemmArgs a) {
   static_assert(ST >= 2 && ST <= 8 && BM >= 16 && BM <= 64 && (EPI != OP_LMH || BM == 16), "ring GEMM shape");
   using R = OpRing<FMT, BM>;
   const OpHdr hd = op_hdr(a.c);
@@ -544,8 +563,8 @@ __global__ __launch_bounds__(256) void op_gemm_ring_kernel(OpGemmArgs a) {
   constexpr int TM = BM / 16;
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
   const int kg = lane >> 4, n = lane & 15;
-  // (tiles renumbered per XCD for the 32- and 64-row prefill tiles but gate/up, as
-  // op_gemm_kernel; the argmax epilogue indexes by blockIdx.x)
+  // (tiles renumbered per XCD for the 32- and 64-row prompt tiles but gate/up, which was no faster
+  // that way; the argmax epilogue indexes by blockIdx.x)
   const OpTile tl = EPI != OP_SILU && BM > 16 ? op_tile_xcd() : OpTile{(int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z};
   const int n0 = tl.x * OP_BN, m0 = tl.y * BM;
   const int K = a.W.K, qg = a.W.qg;
@@ -593,12 +612,16 @@ __global__ __launch_bounds__(256) void op_gemm_ring_kernel(OpGemmArgs a) {
     }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no LDS load outlives the workgroup
   if constexpr (EPI == OP_QKV) op_gemm_epilogue<BM, EPI>(a, hd, acc, m0, n0, tl.z, w, kg, n, red, a.pos_hint, qcs, qbias);
-  else op_gemm_epilogue<BM, EPI>(a, hd, acc, m0, n0, tl.z, w, kg, n, red);
+  else {
+    if (EPI == OP_SILU) lds_barrier();   // the ring's stages become the epilogue's tile
+    static_assert(EPI != OP_SILU || R::N * 16 >= BM * OP_HLD * 2, "a stage holds the tile");
+    op_gemm_epilogue<BM, EPI>(a, hd, acc, m0, n0, tl.z, w, kg, n, red, -1, nullptr, nullptr, (uint16_t*)r0);
+  }
 }
 
 // Residual split-K reduction fused with the RMSNorm that reads the updated residual, for
 // passes of up to 16 rows: one workgroup per row m, one thread per column. x[m] += the
-// slices' partials (added in slice order, as op_epi_kernel); then, for rows m >= row0,
+// slices' partials (added in slice order); then, for rows m >= row0,
 // xn[m - row0] = f16(x * rsqrt(mean(x^2) + eps) * gamma), the sum of squares taken per wave
 // and the 14 wave sums added in order (a function of the row alone, so 1-row and 16-row
 // passes agree bit for bit).

@@ -862,25 +862,8 @@ struct KVFrag {
   uint4 v[4][2];
 };
 
-// SWZ: the cache in the swizzled layout of the q8 / f16 engines (ill_common.h; the same
-// fragments, read as 256-byte runs); the pass kernel's cache is in rows.
-template <bool SWZ = false>
 __device__ __forceinline__ void kv_fetch(const uint16_t* kbase, const uint16_t* vbase, int c, int lane, KVFrag& f) {
   const int kg = lane >> 4, n = lane & 15;
-  if constexpr (SWZ) {
-#pragma unroll
-    for (int b = 0; b < 4; b++) {
-      f.k[b][0] = gld((const uint4*)(kbase + kv_k_off(64 * c + 16 * b + n, 8 * kg, true)));
-      f.k[b][1] = gld((const uint4*)(kbase + kv_k_off(64 * c + 16 * b + n, 32 + 8 * kg, true)));
-    }
-#pragma unroll
-    for (int nb = 0; nb < 4; nb++) {
-#pragma unroll
-      for (int ks = 0; ks < 2; ks++)
-        f.v[nb][ks] = gld((const uint4*)(vbase + kv_v_off(64 * c + 32 * ks + 8 * kg, 16 * nb + n, true)));
-    }
-    return;
-  }
 #pragma unroll
   for (int b = 0; b < 4; b++) {
     const uint4* kr = (const uint4*)(kbase + (size_t)(64 * c + 16 * b + n) * 64);
