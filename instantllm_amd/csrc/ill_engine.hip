@@ -347,14 +347,9 @@ bool op_gemm(ill_engine* e, const __half* A, const OpMat& W, int M, int layer, c
     const int mt = (M + 63) / 64;
     int S = 1;
     if constexpr (EPI == OP_RESID) {
-      // K slices: as many as put about one tile on every CU; three where that puts up to two
-      // tiles on every CU (129-170 tiles; 1500 rows: whole prompts 3.30 -> 2.94 ms
-      // q4, 3.45 -> 3.03 q8, 3.26 -> 3.00 f16; at 2000 and 3000 rows splitting gained nothing)
-      const int tiles = ntn * mt, cap = (int)(ILL_OP_PART_BYTES / ((size_t)M * W.N * 4));   // partial buffer
-      S = tiles > 128 && 3 * tiles <= 512 ? 3 : std::max(1, 256 / tiles);
-      S = std::max(1, std::min(std::min(S, nsteps / 4), std::min(OP_MAXS, cap)));
+      const int cap = (int)(ILL_OP_PART_BYTES / ((size_t)M * W.N * 4));   // partial buffer
+      S = op_slices(ntn * mt, nsteps, cap);
       g.ksteps = (nsteps + S - 1) / S;
-      S = (nsteps + g.ksteps - 1) / g.ksteps;
     }
     hipLaunchKernelGGL((op_gemm_ring_kernel<FMT, 64, EPI, OP_RING_ST(FMT, EPI)>), dim3(ntn, mt, S), dim3(256), 0, e->stream, g);
     if (S == 1) return false;

@@ -22,6 +22,7 @@
 // step recorded in a hipGraph replays correctly.
 #pragma once
 #include "ill_pass.h"
+#include "ill_plan.h"
 
 // Rows of a prompt chunk at most (less where the context is shorter). The GEMMs need many rows
 // to fill the chip: whole prompts in chunks of 512 / 1024 / 2048 rows took 16.9 / 13.6 / 11.6 ms
@@ -206,7 +207,6 @@ struct OpGemmArgs {
 #define OP_BN 128
 #define OP_HLD 72    // LDS row stride (halves) of a gate/up tile's hidden units
 #define OP_BK 64
-#define OP_MAXS 24   // K slices of a split GEMM at most
 
 // q8 dequantization, 4 weights at a time: s * (f16)q for the 4 int8 codes of x. Each code
 // q becomes the half 1024 + (q + 128) (exponent 0x64 over the byte q ^ 0x80, built with
