@@ -20,3 +20,11 @@ constexpr int op_slices(int tiles, int nsteps, int cap) {
   const int per = (nsteps + s - 1) / s;
   return (nsteps + per - 1) / per;
 }
+
+// 64-position chunks that the attention of a row at pos + dep reads (pos .. the row itself
+// included), never past the cache: a finished request may stand at pos = maxctx, and the passes of
+// 1 to 16 rows still queued behind it compute, without storing, on positions beyond that.
+constexpr int row_chunks(int pos, int dep, int maxctx) {
+  const int n = (pos + dep + 64) >> 6;
+  return n < maxctx / 64 ? n : maxctx / 64;
+}

@@ -213,8 +213,8 @@ __device__ __forceinline__ void row_combine(const float2* o, const float2* ml, i
   y1 = a1 / l;
 }
 // the splits of a row at pos + dep
-__device__ __forceinline__ int row_splits(int pos, int dep) {
-  return __builtin_amdgcn_readfirstlane(min(ROW_NSPLIT, (((pos + dep + 64) >> 6) + 7) >> 3));
+__device__ __forceinline__ int row_splits(const OpCtx& c, int pos, int dep) {
+  return __builtin_amdgcn_readfirstlane(min(ROW_NSPLIT, (row_chunks(pos, dep, c.maxctx) + 7) >> 3));
 }
 
 // Attention: a workgroup per (row, KV group, split j < nsplit) takes the splits j, j + nsplit, ..;
@@ -286,7 +286,7 @@ __global__ __launch_bounds__(64 * ILL_WAVES) void row_attn_kernel(OpCtx c, int l
   const int pos = hd.pos;
   const bool tree = hd.mode == ILL_MODE_TREE;
   const int dep = tree ? dp0 : (hd.mode == ILL_MODE_DECODE ? 0 : t);
-  const int L = pos + dep + 1, nch = (L + 63) >> 6;
+  const int L = pos + dep + 1, nch = row_chunks(pos, dep, c.maxctx);
   const int nne = min(ROW_NSPLIT, (nch + 7) >> 3);
   if (tree) {   // the row's ancestors by depth, from the parents held by lanes 0-15
     int pr = tl, r = __builtin_amdgcn_readfirstlane(t);
@@ -470,7 +470,7 @@ __global__ __launch_bounds__(256) void row_comb_kernel(OpCtx c, const float* att
   }
   const int dep = hd.mode == ILL_MODE_TREE ? dp : (hd.mode == ILL_MODE_DECODE ? 0 : t);
   float y, unused;
-  row_combine(o, ml, row_splits(hd.pos, dep), y, unused);
+  row_combine(o, ml, row_splits(c, hd.pos, dep), y, unused);
   if (!hd.done) gst((uint16_t*)(c.ao + (size_t)rh * 64 + lane), (uint16_t)__half_as_ushort(__float2half(y)));
 }
 
@@ -519,7 +519,7 @@ __global__ __launch_bounds__(448) void row_o_kernel(OpCtx c, OpMat W, const floa
     fetch();
     const int dp = gld(c.tree + ILL_TR_DEPTH);
     __builtin_amdgcn_sched_barrier(0);
-    const int nne = row_splits(hd.pos, hd.mode == ILL_MODE_TREE ? dp : 0);
+    const int nne = row_splits(c, hd.pos, hd.mode == ILL_MODE_TREE ? dp : 0);
     if (nne > nsplit) states(nsplit, nne);
     float y0, y1;
     row_combine(o, q, nne, y0, y1);

@@ -133,3 +133,37 @@ def test_prompt_attention_shapes(fmt, tmp_path):
             assert metrics.rel_l2(e.read_logits(0), ref) <= REL_L2_TOL, parts
     finally:
         e.close()
+
+
+@pytest.mark.parametrize("graph", ["steps", "spec"])
+def test_passes_queued_behind_the_contexts_end(graph, tmp_path):
+    """A chain pass in the last 16 slots of the context, all of its drafts accepted, leaves the
+    request finished at pos = 576 = the context; the 1- and 16-row passes of a captured graph
+    that still run then change nothing, and the next request is right."""
+    from instantllm_amd.engine import Engine
+    path = str(tmp_path / "m.ill")
+    synth.build_model(path, F.FMT_Q8, seed=6, shape=synth.ModelShape(layers=2, vocab=VOCAB))
+    toks = [int(t) for t in np.random.default_rng(760).integers(0, VOCAB, size=560)]
+    with Engine(path, max_context=1024, max_pass=16, max_steps=64) as big:
+        big.set_state(pos=0, n=560, maxsteps=64, eos=NO_EOS)
+        big.prefill(toks, write_logits=True)
+        want = big.read_logits(0)
+        for _ in range(16):
+            big.decode_step()
+        chain = [int(t) for t in big.out_tokens()[:17]]
+    with Engine(path, max_context=576, max_pass=16, max_steps=64) as e:
+        e.set_state(pos=0, n=560, maxsteps=64, eos=NO_EOS, tspec=16)
+        (e.capture_spec if graph == "spec" else e.capture_steps)(2)
+        e.prefill(toks)
+        e.verify_pass(16, toks=chain[:16], write_logits=True)
+        assert int(np.argmax(e.read_logits(15))) == chain[16]
+        st, kv = e.get_state(), e.kv_copy_out(576)
+        assert st["done"] and st["pos"] == 576
+        print("finished at the context's end, launching", graph, flush=True)
+        e.launch_graph()
+        e.sync()
+        assert e.get_state() == st
+        assert all(np.array_equal(a, b) for a, b in zip(kv, e.kv_copy_out(576)))
+        e.set_state(pos=0, n=560, maxsteps=64, eos=NO_EOS)
+        e.prefill(toks, write_logits=True)
+        assert np.array_equal(e.read_logits(0).view(np.uint32), want.view(np.uint32))

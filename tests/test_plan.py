@@ -49,3 +49,22 @@ def test_k_slices_of_prompt_products(tmp_path, k):
     per = -(-nsteps // s)
     assert ((s - 1) * per < nsteps).all() and (s * per >= nsteps).all()
     assert (s * m * H * 4 <= PART_BYTES)[s > 1].all()
+
+
+def test_attention_chunks_stay_inside_the_cache(tmp_path):
+    """Every row of a live pass reads all of its positions; a row of a pass queued behind a request
+    that ended at the context's limit reads no chunk past the cache."""
+    t = evaluate(tmp_path, """
+      for (int ctx = 64; ctx <= 4608; ctx += ctx < 1024 ? 64 : 512)
+        for (int pos = 0; pos <= ctx; pos++)
+          for (int dep = 0; dep < 16; dep += 5) printf("%d %d %d %d\\n", ctx, pos, dep, row_chunks(pos, dep, ctx));""")
+    ctx, pos, dep, n = t.T
+    assert (64 * n <= ctx).all()
+    live = pos + 16 <= ctx
+    assert np.array_equal(n[live], -(-(pos + dep + 1)[live] // 64))
+    assert (n >= 1).all()
+
+
+def test_row_attention_takes_its_chunks_from_the_plan():
+    text = (CSRC / "ill_rows.h").read_text()
+    assert "nch = row_chunks(pos, dep, c.maxctx);" in text
