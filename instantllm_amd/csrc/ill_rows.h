@@ -222,9 +222,15 @@ __device__ __forceinline__ int row_splits(const OpCtx& c, int pos, int dep) {
 // group's seven heads at once: the heads are columns of the MFMA blocks (scores: K rows x heads,
 // then V dims x heads), so K and V are read once per group, softmax statistics are per lane, and
 // P needs no cross-lane move (the key of block b, row 4 kg + r is 32 (b / 2) + 8 kg + 4 (b % 2) + r,
-// so a lane's scores are the eight consecutive keys of its operand slots). q and P are split into
-// f16 high and low parts (fp32-accurate products). The waves' states are combined in wave order
-// into the split's state, the row's splits in split order: here with nsplit = 1 (c.ao gets the
+// so a lane's scores are the eight consecutive keys of its operand slots). q and P enter
+// the products as f16 pairs (high, low) that keep fp32's precision: q scaled by the power of two
+// that brings the row and head's largest dim to f16's range, P by 2^15 and its low part by a
+// further 2^11, into sums of its own. Unscaled pairs end in f16's subnormals (2^-25 absolute).
+// Errors against 64 bits over the products' 2-norm, fp32 FMA chain / unscaled / these, in units of
+// 2^-23: scores at |q| ~ 1, 0.1, 0.01: 1.2 / 1.4 / 0.8, 1.2 / 12 / 0.8, 1.2 / 121 / 0.8; P V with
+// the scores spread over 5, 10 in log2: 1.2 / 4.6 / 0.7, 1.0 / 11 / 0.7. The scaling costs 0.5-1% of a
+// pass (nine 1-row q8 steps 5.24 -> 5.29 ms after 500 positions, 5.50 -> 5.55 after 4000).
+// The waves' states are combined in wave order into the split's state, the row's splits in split order: here with nsplit = 1 (c.ao gets the
 // f16 output), else by the readers of att (row_o_kernel for one row, row_comb_kernel), with the
 // same arithmetic, so the launch's split does not change the result.
 // One chunk per wave up to 512 nsplit positions; 512 positions of 1 row take 2 workgroups.
@@ -271,17 +277,40 @@ __global__ __launch_bounds__(64 * ILL_WAVES) void row_attn_kernel(OpCtx c, int l
     vload(ch);
   }
   __builtin_amdgcn_sched_barrier(0);
+  // over the lane groups kg (the head's other keys or dims)
+  auto over_kg = [](float v, auto op) {
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_int(v), __float_as_int(v), false, false);
+    v = op(__int_as_float((int)a[0]), __int_as_float((int)a[1]));
+    const auto q = __builtin_amdgcn_permlane32_swap(__float_as_int(v), __float_as_int(v), false, false);
+    return op(__int_as_float((int)q[0]), __int_as_float((int)q[1]));
+  };
+  // q as f16 pairs of q 2^(15 - e), whose largest dim fills f16's range, and the power of two
+  // that takes the scores back (with the 1 / 8)
   v8h qh[2], ql[2];
+  float qback;
+  {
+    float v[2][8], mx = 0.f;
 #pragma unroll
-  for (int ks = 0; ks < 2; ks++) {
-    const float v[8] = {qf[ks][0].x, qf[ks][0].y, qf[ks][0].z, qf[ks][0].w, qf[ks][1].x, qf[ks][1].y, qf[ks][1].z, qf[ks][1].w};
+    for (int ks = 0; ks < 2; ks++) {
+      const float x[8] = {qf[ks][0].x, qf[ks][0].y, qf[ks][0].z, qf[ks][0].w, qf[ks][1].x, qf[ks][1].y, qf[ks][1].z, qf[ks][1].w};
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-      const float x = v[i] * 0.125f;
-      const _Float16 hi = (_Float16)x;
-      qh[ks][i] = hi;
-      ql[ks][i] = (_Float16)(x - (float)hi);
+      for (int i = 0; i < 8; i++) {
+        v[ks][i] = x[i];
+        mx = fmaxf(mx, fabsf(x[i]));
+      }
     }
+    const int e = max(__builtin_amdgcn_frexp_expf(over_kg(mx, OpMaxF{})), -100);
+    const float up = __builtin_ldexpf(1.f, 15 - e);
+    qback = __builtin_ldexpf(0.125f, e - 15);
+#pragma unroll
+    for (int ks = 0; ks < 2; ks++)
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+        const float x = v[ks][i] * up;
+        const _Float16 hi = (_Float16)x;
+        qh[ks][i] = hi;
+        ql[ks][i] = (_Float16)(x - (float)hi);
+      }
   }
   const int pos = hd.pos;
   const bool tree = hd.mode == ILL_MODE_TREE;
@@ -361,17 +390,10 @@ __global__ __launch_bounds__(64 * ILL_WAVES) void row_attn_kernel(OpCtx c, int l
         const int vp = 64 * ch + 32 * (b >> 1) + 8 * kg + 4 * (b & 1);
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-          sc[b][r] = vp + r < L ? d[r] : -INFINITY;
+          sc[b][r] = vp + r < L ? d[r] * qback : -INFINITY;
           mc = fmaxf(mc, sc[b][r]);
         }
       }
-      // over the lane groups kg (the head's other keys)
-      auto over_kg = [](float v, auto op) {
-        const auto a = __builtin_amdgcn_permlane16_swap(__float_as_int(v), __float_as_int(v), false, false);
-        v = op(__int_as_float((int)a[0]), __int_as_float((int)a[1]));
-        const auto q = __builtin_amdgcn_permlane32_swap(__float_as_int(v), __float_as_int(v), false, false);
-        return op(__int_as_float((int)q[0]), __int_as_float((int)q[1]));
-      };
       mc = over_kg(mc, OpMaxF{});
       float lc = 0.f;
       v8h ph[2], pl[2];
@@ -379,24 +401,25 @@ __global__ __launch_bounds__(64 * ILL_WAVES) void row_attn_kernel(OpCtx c, int l
       for (int b = 0; b < 4; b++)
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-          const float p = att_exp(sc[b][r] - mc);
+          const float p = att_exp(sc[b][r] - mc), x = p * 32768.f;   // p <= 1
           lc += p;
-          const _Float16 hi = (_Float16)p;
+          const _Float16 hi = (_Float16)x;
           ph[b >> 1][4 * (b & 1) + r] = hi;
-          pl[b >> 1][4 * (b & 1) + r] = (_Float16)(p - (float)hi);
+          pl[b >> 1][4 * (b & 1) + r] = (_Float16)((x - (float)hi) * 2048.f);
         }
       lc = over_kg(lc, OpAddF{});
       const AttScale k = att_scale(Mx, mc);
+      const float sb = k.sb * 0x1p-15f;
 #pragma unroll
       for (int nb = 0; nb < 4; nb++) {
-        v4f d = {0.f, 0.f, 0.f, 0.f};
+        v4f d = {0.f, 0.f, 0.f, 0.f}, dl = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int q = 0; q < 2; q++) {
           d = __builtin_amdgcn_mfma_f32_16x16x32_f16(u4_to_v8h(vf[nb][q]), ph[q], d, 0, 0, 0);
-          d = __builtin_amdgcn_mfma_f32_16x16x32_f16(u4_to_v8h(vf[nb][q]), pl[q], d, 0, 0, 0);
+          dl = __builtin_amdgcn_mfma_f32_16x16x32_f16(u4_to_v8h(vf[nb][q]), pl[q], dl, 0, 0, 0);
         }
 #pragma unroll
-        for (int r = 0; r < 4; r++) O[nb][r] = att_fold(O[nb][r], d[r], k);
+        for (int r = 0; r < 4; r++) O[nb][r] = O[nb][r] * k.sa + fmaf(dl[r], 0x1p-11f, d[r]) * sb;
       }
       Ls = att_fold(Ls, lc, k);
       Mx = k.mn;

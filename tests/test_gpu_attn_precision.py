@@ -1,0 +1,90 @@
+"""Attention of passes of up to 16 rows (q8 / f16) keeps fp32 queries and probabilities: caches on
+which operands of 16 bits, or pairs of them whose low halves run into f16's subnormals, show in
+the logits. The attention norm of a one-layer model is set to zero, so that q is the QKV bias
+(fp32, no activation rounding) and the row's own key and value are zero; keys and values are
+written into the cache. Logits against the oracle in float64, relative L2 <= 1.5e-3: the f16
+roundings of the attention output, of the MLP's input and of its hidden units (2^-12 each, rms
+1.4e-4) leave 3e-4 to 6e-4. (Pairs of unscaled
+values: 2e-3 to 9e-3.)"""
+from __future__ import annotations
+
+import struct
+
+import numpy as np
+import pytest
+
+from instantllm_amd import illfile as F, synth
+from oracle import illread, metrics, qwen
+
+pytestmark = pytest.mark.gpu
+VOCAB, CTX, NO_EOS = 1024, 2176, (-5, -5)
+REL_L2_TOL = 1.5e-3
+
+
+@pytest.fixture(scope="module", params=[F.FMT_Q8, F.FMT_F16], ids=["q8", "f16"])
+def base(request, tmp_path_factory):
+    path = str(tmp_path_factory.mktemp("att") / "m.ill")
+    synth.build_model(path, request.param, seed=9, shape=synth.ModelShape(layers=1, vocab=VOCAB))
+    return path
+
+
+def patched(base, tmp_path, bq):
+    """The model with ln1 = 0 and the QKV bias (bq, 0, 0)."""
+    path = str(tmp_path / "p.ill")
+    data = bytearray(open(base, "rb").read())
+    count = struct.unpack_from("<I", data, 12)[0]
+    tab = np.frombuffer(bytes(data[16:16 + 16 * count]), "<u8").reshape(count, 2)
+    bias = np.concatenate([bq.reshape(-1), np.zeros(256)])[F.qkv_row_order()].astype("<f4").tobytes()
+    for tid, val in ((F.layer_id(0, F.ATTN_NORM), bytes(4 * 896)), (F.layer_id(0, F.BQKV), bias)):
+        off, size = (int(x) for x in tab[tid])
+        assert size == len(val)
+        data[off:off + size] = val
+    open(path, "wb").write(data)
+    return path
+
+
+def check(path, pos, k, v):
+    """k, v: f16 [2, pos, 64]. The logits of one row at pos against the float64 oracle."""
+    from instantllm_amd.engine import Engine
+    m = qwen.Model(illread.load(path), dtype=np.float64)
+    cache = m.new_cache(pos + 1)
+    cache.k[0][:, :pos], cache.v[0][:, :pos], cache.len = k, v, pos
+    ref = m.forward([7], cache)
+    with Engine(path, max_context=CTX, max_pass=16, max_steps=16) as e:
+        e.kv_copy_in(k[None].view(np.uint16), v[None].view(np.uint16))
+        e.set_state(pos=pos, n=1, maxsteps=16, eos=NO_EOS)
+        e.prefill([7], write_logits=True)
+        got = e.read_logits(0)
+    err = metrics.rel_l2(got, ref)
+    print("rel_l2", err, flush=True)
+    assert err <= REL_L2_TOL
+
+
+def rope(x, pos):
+    c, s = qwen.rope_cos_sin(np.array([pos]), np.float64)
+    return x * c + qwen.rotate_half(x) * s
+
+
+@pytest.mark.parametrize("pos", [300, 700, 2100])
+def test_small_probabilities_beside_a_sink(base, tmp_path, pos):
+    """One key takes nearly all of the weight and has no value; the output is the sum of the
+    chunk's other probabilities of 2^-19 to 2^-21 (a level per head) times large values."""
+    rng = np.random.default_rng(pos)
+    u = rng.standard_normal(64)
+    level = 19 + 2 * np.arange(14) / 13
+    bq = u[None] * level[:, None] / level.mean()
+    r = rope(u, pos)[0]
+    k = np.zeros((2, pos, 64), np.float16)
+    k[:, 3] = (r * 8 * level.mean() * np.log(2) / (r @ r)).astype(np.float16)
+    v = np.broadcast_to((3e4 * rng.uniform(-1, 1, size=(2, 1, 64))).astype(np.float16), k.shape).copy()
+    v[:, 3], v[:, 64:] = 0, 0   # (another chunk's probabilities are relative to its own largest)
+    check(patched(base, tmp_path, bq), pos, k, v)
+
+
+@pytest.mark.parametrize("pos", [300, 700, 2100])
+def test_small_queries_against_large_keys(base, tmp_path, pos):
+    rng = np.random.default_rng(pos)
+    bq = 1.5e-4 * rng.standard_normal((14, 64))
+    k = (6e4 * rng.uniform(-1, 1, size=(2, pos, 64))).astype(np.float16)
+    v = rng.standard_normal((2, pos, 64)).astype(np.float16)
+    check(patched(base, tmp_path, bq), pos, k, v)
