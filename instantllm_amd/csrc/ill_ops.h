@@ -672,7 +672,7 @@ __device__ __forceinline__ void att_combine(const float* m, const float* l, cons
   oo = acc;
 }
 
-#define OP_ATTN_LAG 8.0f
+#define OP_ATTN_UP 14.0f   // log2 of the largest probability (of its share of f16's range)
 // ---- attention of prompt chunks of more than 16 rows: MFMA flash attention ----------------
 // A wave evaluates 16 rows of one query head against 64-position chunks of the cache (this
 // chunk's QKV kernel has written its own keys and values): row t < M sits at position pos + t and
@@ -681,7 +681,7 @@ __device__ __forceinline__ void att_combine(const float* m, const float* l, cons
 // MFMA block are dealt out (block b, row 4 kg + r: key 32 (b / 2) + 8 kg + 4 (b % 2) + r) such
 // that the probabilities a lane holds are the next product's operand as they stand: no pass
 // through LDS, no reduction across the 16 lanes of a row. q and P are split into f16 high and
-// low parts (products as accurate as fp32 q and P). The sums of the exponentials stay per lane
+// low parts. The sums of the exponentials stay per lane
 // until the end, and the value products accumulate onto the output. The next chunk streams in
 // meanwhile. The kernel is bound by the vector instructions per score.
 // GRP: a workgroup per (16 rows, four or three heads of a KV group), SPL waves per head taking turns
@@ -690,7 +690,8 @@ __device__ __forceinline__ void att_combine(const float* m, const float* l, cons
 // wave order. 2000 rows from position 0: 61 us per layer (q4 79) with scores as rows x keys and P
 // turned through LDS, every head reading K and V itself; 40 (101) with the layout above, 44 (45)
 // with chunks shared through LDS by seven heads, 37 (39) with two waves per head and the lazy
-// maximum, 29 (30) with the heads on two workgroups, so that the causal load evens out.
+// maximum, 29 (30) with the heads on two workgroups, so that the causal load evens out; 30.5 since the
+// probabilities fill f16's range.
 template <bool SWZ, bool GRP, int SPL>   // SWZ: the K/V cache layout (ill_common.h): swizzled for q8 / f16, rows for q4
 __global__ __launch_bounds__(64 * SPL * (GRP ? 4 : 1), GRP ? 1 : 2) void op_attn_rows_kernel(OpCtx c, int layer, int M, int blk0) {
   const OpHdr hd = op_hdr(c);
@@ -736,21 +737,28 @@ __global__ __launch_bounds__(64 * SPL * (GRP ? 4 : 1), GRP ? 1 : 2) void op_attn
     const auto q = __builtin_amdgcn_permlane32_swap(__float_as_int(v), __float_as_int(v), false, false);
     return op(__int_as_float((int)q[0]), __int_as_float((int)q[1]));
   };
-  v8h qh[2], ql[2];   // q / 8 * log2(e): the scores are exponents of 2
+  // q / 8 * log2(e) as f16 pairs, of the product before its rounding to fp32: the scores are
+  // exponents of 2
+  constexpr float LG = 1.4426950408889634f, LGL = (float)(1.4426950408889634 - (double)LG);
+  v8h qh[2], ql[2];
 #pragma unroll
   for (int ks = 0; ks < 2; ks++) {
     const float v[8] = {qf[ks][0].x, qf[ks][0].y, qf[ks][0].z, qf[ks][0].w, qf[ks][1].x, qf[ks][1].y, qf[ks][1].z, qf[ks][1].w};
 #pragma unroll
     for (int i = 0; i < 8; i++) {
-      const float x = v[i] * (0.125f * 1.4426950408889634f);
+      const float q8 = v[i] * 0.125f, x = q8 * LG;
       const _Float16 hi = (_Float16)x;
       qh[ks][i] = hi;
-      ql[ks][i] = (_Float16)(x - (float)hi);
+      ql[ks][i] = (_Float16)((x - (float)hi) + fmaf(q8, LGL, fmaf(q8, LG, -x)));
     }
   }
-  // The exponents' reference Mx of a row follows its maximum lazily: the score products start from
-  // -Mx, and only when a score comes out above OP_ATTN_LAG is Mx moved up and everything summed so
-  // far rescaled (p <= 2^OP_ATTN_LAG stays far inside f16 and fp32). The first chunk sets it.
+  // The exponents' reference Mx of a row follows its maximum lazily, OP_ATTN_UP below it: the first
+  // chunk sets it, and only when a score exceeds the row's by more than 1 is it moved up and
+  // everything summed so far rescaled. Probabilities then reach 2^14 to 2^15, so that their f16
+  // pairs hold 24 bits down to 2^-15 of the largest. (With the reference at the maximum and moved at
+  // 8, chunks far below it lost half of their bits to f16's subnormals.) The score products start
+  // from 0 and the reference is subtracted: started from -Mx the exponents' error is up to 1.8
+  // times as large. Both together cost 28.0 -> 30.5 us per layer at 2000 rows.
   float Mx = 0.f, Ls = 0.f;   // Ls: this lane's keys only
   bool first = true;
   v4f O[4];
@@ -760,7 +768,7 @@ __global__ __launch_bounds__(64 * SPL * (GRP ? 4 : 1), GRP ? 1 : 2) void op_attn
     v4f sc[4];
 #pragma unroll
     for (int b = 0; b < 4; b++) {
-      v4f d = {-Mx, -Mx, -Mx, -Mx};
+      v4f d = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int ks = 0; ks < 2; ks++) {
         d = __builtin_amdgcn_mfma_f32_16x16x32_f16(u4_to_v8h(f.k[b][ks]), qh[ks], d, 0, 0, 0);
@@ -780,26 +788,24 @@ __global__ __launch_bounds__(64 * SPL * (GRP ? 4 : 1), GRP ? 1 : 2) void op_attn
     for (int b = 0; b < 4; b++)
 #pragma unroll
       for (int r = 0; r < 4; r++) mc = fmaxf(mc, sc[b][r]);
-    if (first || __any(mc > OP_ATTN_LAG)) {   // (wave-uniform)
+    if (first || __any(mc > Mx + (OP_ATTN_UP + 1.f))) {   // (wave-uniform)
       mc = over_kg(mc, OpMaxF{});
-      // up by the excess; the first chunk: to the maximum (a row with no position in it stays at 0)
-      const float up = first ? (mc == -INFINITY ? 0.f : mc) : fmaxf(mc, 0.f);
-      // (nothing is summed before the first chunk, whose maximum may be far below 0: 0 * 2^-up would be NaN)
-      const float sa = first ? 1.f : __builtin_amdgcn_exp2f(-up);
+      // (a row with no position in its first chunk stays at 0)
+      const float mn = first ? (mc == -INFINITY ? 0.f : mc - OP_ATTN_UP) : fmaxf(mc - OP_ATTN_UP, Mx);
+      // (nothing is summed before the first chunk, whose maximum may be far below 0: 0 * 2^-mn would be NaN)
+      const float sa = first ? 1.f : __builtin_amdgcn_exp2f(Mx - mn);
       first = false;
-      Mx += up;
+      Mx = mn;
       Ls *= sa;
 #pragma unroll
       for (int nb = 0; nb < 4; nb++) O[nb] *= sa;
-#pragma unroll
-      for (int b = 0; b < 4; b++) sc[b] -= up;
     }
     v8h ph[2], pl[2];
 #pragma unroll
     for (int b = 0; b < 4; b++)
 #pragma unroll
       for (int r = 0; r < 4; r += 2) {
-        const float p0 = __builtin_amdgcn_exp2f(sc[b][r]), p1 = __builtin_amdgcn_exp2f(sc[b][r + 1]);
+        const float p0 = __builtin_amdgcn_exp2f(sc[b][r] - Mx), p1 = __builtin_amdgcn_exp2f(sc[b][r + 1] - Mx);
         Ls += p0;
         Ls += p1;
         const _Float16 h0 = (_Float16)p0, h1 = (_Float16)p1;
@@ -892,12 +898,11 @@ __global__ __launch_bounds__(64 * SPL * (GRP ? 4 : 1), GRP ? 1 : 2) void op_attn
       for (int nb = 0; nb < 4; nb++) O[nb] = O[nb] * e0 + *(const v4f*)&st[128 + 256 * nb + 4 * lane] * e1;
     }
     if (hd.done || !live || t0 + n >= M) return;
-    const float inv = 1.0f / Ls;
 #pragma unroll
     for (int nb = 0; nb < 4; nb++) {
       uint2 y;
-      y.x = f2h(O[nb][0] * inv) | (f2h(O[nb][1] * inv) << 16);
-      y.y = f2h(O[nb][2] * inv) | (f2h(O[nb][3] * inv) << 16);
+      y.x = f2h(O[nb][0] / Ls) | (f2h(O[nb][1] / Ls) << 16);
+      y.y = f2h(O[nb][2] / Ls) | (f2h(O[nb][3] / Ls) << 16);
       gst((gu32x2*)(c.ao + (size_t)t * ILL_H + h * 64 + 16 * nb + 4 * kg), (gu32x2){y.x, y.y});
     }
   } else {
