@@ -681,12 +681,13 @@ __device__ __forceinline__ void att_combine(const float* m, const float* l, cons
 // MFMA block are dealt out (block b, row 4 kg + r: key 32 (b / 2) + 8 kg + 4 (b % 2) + r) such
 // that the probabilities a lane holds are the next product's operand as they stand: no pass
 // through LDS, no reduction across the 16 lanes of a row. q and P are split into f16 high and
-// low parts. The sums of the exponentials stay per lane
-// until the end, and the value products accumulate onto the output. The next chunk streams in
-// meanwhile. The kernel is bound by the vector instructions per score.
+// low parts. The sums of the exponentials stay per lane until the end, and the value products
+// accumulate onto the output. The next chunk streams in meanwhile. The kernel is bound by the vector
+// instructions per score.
 // GRP: a workgroup per (16 rows, four or three heads of a KV group), SPL waves per head taking turns
 // at the chunks; SPL chunks' keys and values at a time go from memory straight into LDS once for
-// the heads (16 KB each, two buffers: the next ones stream in meanwhile). For few blocks (GRP false): SPL waves per (16 rows, query head), chunk c to wave c % SPL, their states combined in
+// the heads (16 KB each, two buffers: the next ones stream in meanwhile). For few blocks (GRP
+// false): SPL waves per (16 rows, query head), chunk c to wave c % SPL, their states combined in
 // wave order. 2000 rows from position 0: 61 us per layer (q4 79) with scores as rows x keys and P
 // turned through LDS, every head reading K and V itself; 40 (101) with the layout above, 44 (45)
 // with chunks shared through LDS by seven heads, 37 (39) with two waves per head and the lazy
@@ -737,21 +738,31 @@ __global__ __launch_bounds__(64 * SPL * (GRP ? 4 : 1), GRP ? 1 : 2) void op_attn
     const auto q = __builtin_amdgcn_permlane32_swap(__float_as_int(v), __float_as_int(v), false, false);
     return op(__int_as_float((int)q[0]), __int_as_float((int)q[1]));
   };
-  // q / 8 * log2(e) as f16 pairs, of the product before its rounding to fp32: the scores are
-  // exponents of 2
+  // q * log2(e) as f16 pairs (of the product before its rounding to fp32), scaled by the power of two
+  // that brings the row's largest dim to f16's range; scores * qback are exponents of 2 (row_attn_kernel)
   constexpr float LG = 1.4426950408889634f, LGL = (float)(1.4426950408889634 - (double)LG);
   v8h qh[2], ql[2];
+  float v[2][8], qm = 0.f;
 #pragma unroll
   for (int ks = 0; ks < 2; ks++) {
-    const float v[8] = {qf[ks][0].x, qf[ks][0].y, qf[ks][0].z, qf[ks][0].w, qf[ks][1].x, qf[ks][1].y, qf[ks][1].z, qf[ks][1].w};
+    const float x[8] = {qf[ks][0].x, qf[ks][0].y, qf[ks][0].z, qf[ks][0].w, qf[ks][1].x, qf[ks][1].y, qf[ks][1].z, qf[ks][1].w};
 #pragma unroll
     for (int i = 0; i < 8; i++) {
-      const float q8 = v[i] * 0.125f, x = q8 * LG;
-      const _Float16 hi = (_Float16)x;
-      qh[ks][i] = hi;
-      ql[ks][i] = (_Float16)((x - (float)hi) + fmaf(q8, LGL, fmaf(q8, LG, -x)));
+      v[ks][i] = x[i];
+      qm = fmaxf(qm, fabsf(x[i]));
     }
   }
+  const int qe = max(__builtin_amdgcn_frexp_expf(over_kg(qm, OpMaxF{})), -100);
+  const float qup = __builtin_ldexpf(1.f, 15 - qe), qback = __builtin_ldexpf(0.125f, qe - 15);
+#pragma unroll
+  for (int ks = 0; ks < 2; ks++)
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      const float y = v[ks][i] * qup, x = y * LG;
+      const _Float16 hi = (_Float16)x;
+      qh[ks][i] = hi;
+      ql[ks][i] = (_Float16)((x - (float)hi) + fmaf(y, LGL, fmaf(y, LG, -x)));
+    }
   // The exponents' reference Mx of a row follows its maximum lazily, OP_ATTN_UP below it: the first
   // chunk sets it, and only when a score exceeds the row's by more than 1 is it moved up and
   // everything summed so far rescaled. Probabilities then reach 2^14 to 2^15, so that their f16
@@ -788,6 +799,7 @@ __global__ __launch_bounds__(64 * SPL * (GRP ? 4 : 1), GRP ? 1 : 2) void op_attn
     for (int b = 0; b < 4; b++)
 #pragma unroll
       for (int r = 0; r < 4; r++) mc = fmaxf(mc, sc[b][r]);
+    mc *= qback;
     if (first || __any(mc > Mx + (OP_ATTN_UP + 1.f))) {   // (wave-uniform)
       mc = over_kg(mc, OpMaxF{});
       // (a row with no position in its first chunk stays at 0)
@@ -805,7 +817,7 @@ __global__ __launch_bounds__(64 * SPL * (GRP ? 4 : 1), GRP ? 1 : 2) void op_attn
     for (int b = 0; b < 4; b++)
 #pragma unroll
       for (int r = 0; r < 4; r += 2) {
-        const float p0 = __builtin_amdgcn_exp2f(sc[b][r] - Mx), p1 = __builtin_amdgcn_exp2f(sc[b][r + 1] - Mx);
+        const float p0 = __builtin_amdgcn_exp2f(fmaf(sc[b][r], qback, -Mx)), p1 = __builtin_amdgcn_exp2f(fmaf(sc[b][r + 1], qback, -Mx));
         Ls += p0;
         Ls += p1;
         const _Float16 h0 = (_Float16)p0, h1 = (_Float16)p1;

@@ -59,6 +59,25 @@ def check(path, pos, k, v):
     assert err <= REL_L2_TOL
 
 
+def check_prompt(path, k, v, rows, rng):
+    """k, v: f16 [2 layers, 2, 300, 64]. The last row's logits of a prompt of `rows` tokens after them."""
+    from instantllm_amd.engine import Engine
+    m = qwen.Model(illread.load(path), dtype=np.float64)
+    cache = m.new_cache(300 + rows)
+    for l in range(2):
+        cache.k[l][:, :300], cache.v[l][:, :300] = k[l], v[l]
+    cache.len = 300
+    toks = [int(t) for t in rng.integers(0, VOCAB, size=rows)]
+    ref = m.forward(toks, cache)
+    with Engine(path, max_context=CTX, max_pass=16, max_steps=16) as e:
+        e.kv_copy_in(k.view(np.uint16), v.view(np.uint16))
+        e.set_state(pos=300, n=rows, maxsteps=16, eos=NO_EOS)
+        e.prefill(toks, write_logits=True)
+        err = metrics.rel_l2(e.read_logits(0), ref)
+    print("rel_l2", err, flush=True)
+    assert err <= REL_L2_TOL
+
+
 def rope(x, pos):
     c, s = qwen.rope_cos_sin(np.array([pos]), np.float64)
     return x * c + qwen.rotate_half(x) * s
@@ -89,13 +108,34 @@ def test_small_queries_against_large_keys(base, tmp_path, pos):
     check(patched(base, tmp_path, bq), pos, k, v)
 
 
+@pytest.mark.parametrize("pos", [300, 700])
+def test_large_queries_against_small_keys(base, tmp_path, pos):
+    """q / 8 beyond f16's range."""
+    rng = np.random.default_rng(pos)
+    bq = 1e6 * rng.standard_normal((14, 64))
+    k = (2e-5 * rng.uniform(-1, 1, size=(2, pos, 64))).astype(np.float16)
+    v = rng.standard_normal((2, pos, 64)).astype(np.float16)
+    check(patched(base, tmp_path, bq), pos, k, v)
+
+
+@pytest.mark.parametrize("scale", [1e-4, 4e5])
+@pytest.mark.parametrize("fmt,rows", [(F.FMT_Q4, 400), (F.FMT_F16, 150)])
+def test_prompt_queries_small_and_large(tmp_path, fmt, rows, scale):
+    """Prompts with queries of 1e-4 and 4e5, the keys' size inverse."""
+    rng = np.random.default_rng(rows)
+    path = str(tmp_path / "m.ill")
+    synth.build_model(path, fmt, seed=9, shape=synth.ModelShape(layers=2, vocab=VOCAB))
+    path = patched(path, tmp_path, scale * rng.uniform(-1, 1, size=(14, 64)))
+    k, v = rng.uniform(-1, 1, size=(2, 2, 2, 300, 64))
+    check_prompt(path, (6 / scale * k).astype(np.float16), v.astype(np.float16), rows, rng)
+
+
 @pytest.mark.parametrize("fmt,rows", [(F.FMT_Q4, 400), (F.FMT_Q4, 40), (F.FMT_F16, 1200), (F.FMT_F16, 150)])
 def test_prompt_chunks_far_below_the_largest_score(tmp_path, fmt, rows):
     """Prompts on both shapes of the prompt attention (two layers, so that layer 0 runs for every
     row): the first chunk holds a key that takes nearly all of the weight and no values, the
     chunks after it probabilities of 2^-19 to 2^-21 and large values. q lies in dims that the
     rotary embedding hardly turns, so that this holds for every row."""
-    from instantllm_amd.engine import Engine
     path = str(tmp_path / "m.ill")
     synth.build_model(path, fmt, seed=9, shape=synth.ModelShape(layers=2, vocab=VOCAB))
     rng = np.random.default_rng(rows)
@@ -108,17 +148,4 @@ def test_prompt_chunks_far_below_the_largest_score(tmp_path, fmt, rows):
     k, v = np.zeros((2, 2, 2, pos, 64), np.float16)
     k[0, :, 3] = (r * 8 * level.mean() * np.log(2) / (r @ r)).astype(np.float16)
     v[0, :, 64:] = (3e4 * rng.uniform(-1, 1, size=(2, 1, 64))).astype(np.float16)
-    m = qwen.Model(illread.load(path), dtype=np.float64)
-    cache = m.new_cache(pos + rows)
-    for l in range(2):
-        cache.k[l][:, :pos], cache.v[l][:, :pos] = k[l], v[l]
-    cache.len = pos
-    toks = [int(t) for t in rng.integers(0, VOCAB, size=rows)]
-    ref = m.forward(toks, cache)
-    with Engine(path, max_context=CTX, max_pass=16, max_steps=16) as e:
-        e.kv_copy_in(k.view(np.uint16), v.view(np.uint16))
-        e.set_state(pos=pos, n=rows, maxsteps=16, eos=NO_EOS)
-        e.prefill(toks, write_logits=True)
-        err = metrics.rel_l2(e.read_logits(0), ref)
-    print("rel_l2", err, flush=True)
-    assert err <= REL_L2_TOL
+    check_prompt(path, k, v, rows, rng)
