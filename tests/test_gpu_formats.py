@@ -112,7 +112,8 @@ def test_tree_logits_match_oracle(model):
 
 
 def test_long_prefill_chunks(model):
-    """A prompt longer than one 512-row chunk: two layer-by-layer chunks, then decode."""
+    """A prompt of 600 tokens (one layer-by-layer chunk on the ring GEMMs), then decode. Prompts of
+    several chunks: tests/test_gpu_rows.py."""
     fmt, e, m = model
     rng = np.random.default_rng(80 + fmt)
     prompt = [int(t) for t in rng.integers(0, VOCAB, size=600)]
@@ -129,8 +130,8 @@ def test_long_prefill_chunks(model):
 
 @pytest.mark.parametrize("n", [17, 31, 33, 63, 65, 511, 513])
 def test_prefill_chunk_edges(model, n):
-    """Prompt lengths at the edges of the prefill GEMMs' row tiles (16, 32 and 64 rows) and of
-    the 512-row chunk, prefilled in one call and again in two calls whose second chunk starts
+    """Prompt lengths at the edges of the prefill GEMMs' row tiles (16, 32 and 64 rows) and
+    around 512, prefilled in one call and again in two calls whose second one starts
     at a position that is not a multiple of 64 (the QKV epilogue's rotary rows are read for
     pos + row): last-row logits and the first decode step after it against the oracle."""
     fmt, e, m = model

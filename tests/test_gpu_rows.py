@@ -86,9 +86,9 @@ def test_captured_step_replayed_at_a_longer_context(model):
 
 @pytest.mark.parametrize("fmt", [F.FMT_Q4, F.FMT_Q8, F.FMT_F16], ids=["q4", "q8", "f16"])
 def test_prompts_at_the_row_kernels_edges(fmt, tmp_path):
-    """Prompt chunks around the longest one the row kernels take (112 rows) and its 16-row
-    groups, a 1-row last chunk (513 = 512 + 1), and prompts in two calls whose second one is
-    short: last-row logits against the oracle."""
+    """Prompts around the longest one the row kernels take (112 rows) and its 16-row groups, one
+    of 513, and prompts in two calls whose second one is short (for q4 its 1, 3 and 16 rows run
+    on the pass kernel): last-row logits against the oracle."""
     from instantllm_amd.engine import Engine
     path = str(tmp_path / "m.ill")
     synth.build_model(path, fmt, seed=6, shape=synth.ModelShape(layers=2, vocab=VOCAB))
@@ -167,3 +167,34 @@ def test_passes_queued_behind_the_contexts_end(graph, tmp_path):
         e.set_state(pos=0, n=560, maxsteps=64, eos=NO_EOS)
         e.prefill(toks, write_logits=True)
         assert np.array_equal(e.read_logits(0).view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("fmt", [F.FMT_Q4, F.FMT_Q8, F.FMT_F16], ids=["q4", "q8", "f16"])
+def test_prompts_of_two_chunks(fmt, tmp_path):
+    """Prompts past the 4096 rows of a chunk, whose last chunk has 1, 3, 16 and 17 rows: the row
+    kernels' three instantiations (for q4, which runs them on its cache layout, only here) and
+    their split attention states, after a chunk that computes no logits. Last-row logits and the
+    decode step after them against the oracle."""
+    from instantllm_amd.engine import Engine
+    path = str(tmp_path / "m.ill")
+    synth.build_model(path, fmt, seed=6, shape=synth.ModelShape(layers=2, vocab=VOCAB))
+    m = qwen.Model(illread.load(path))
+    toks = [int(t) for t in np.random.default_rng(720 + fmt).integers(0, VOCAB, size=4113)]
+    cache = m.new_cache(4120)
+    for c0 in range(0, 4096, 1024):   # (attention memory)
+        m.forward(toks[c0:c0 + 1024], cache)
+    ref = m.forward(toks[4096:], cache, all_logits=True)
+    with Engine(path, max_context=4224, max_pass=16, max_steps=64) as e:
+        for n in (4097, 4099, 4112, 4113):
+            print("prompt", n, flush=True)
+            e.set_state(pos=0, n=n, maxsteps=64, eos=NO_EOS)
+            e.prefill(toks[:n], write_logits=True)
+            got = e.read_logits(0)
+            assert metrics.rel_l2(got, ref[n - 4097]) <= REL_L2_TOL, n
+            tok = int(e.out_tokens()[0])
+            assert tok == int(np.argmax(got))
+            e.decode_step(write_logits=True)
+            cache.len = n
+            assert metrics.rel_l2(e.read_logits(0), m.forward([tok], cache)) <= REL_L2_TOL, n
+            cache.len = n
+            m.forward([toks[n]] if n < 4113 else [0], cache)   # the prompt's own token back in its slot
