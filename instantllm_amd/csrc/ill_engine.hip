@@ -355,7 +355,7 @@ bool op_gemm(ill_engine* e, const __half* A, const OpMat& W, int M, int layer, c
     }
     hipLaunchKernelGGL((op_gemm_ring_kernel<FMT, 64, EPI, OP_RING_ST(FMT, EPI)>), dim3(ntn, mt, S), dim3(256), 0, e->stream, g);
     if (S == 1) return false;
-    hipLaunchKernelGGL(op_epi_norm_kernel, dim3(M), dim3(ILL_H), 0, e->stream, g, S, norm_gamma, 0);
+    hipLaunchKernelGGL(op_epi_norm_kernel, dim3(M), dim3(ILL_H), 0, e->stream, g, S, norm_gamma);
     return true;
   }
 }

@@ -15,8 +15,9 @@
 // Arithmetic: activations in f16 (the reference's G3 path keeps fp16 activations too),
 // weights dequantized to f16 (q4: s*q + m; q8: s*q; f16: as stored),
 // v_mfma_f32_16x16x32_f16 with fp32 accumulation over K in a fixed order, fp32 residual
-// stream. A row's arithmetic does not depend on the rows beside it; passes of up to 16 rows all
-// run on the row kernels, so a row decoded alone and inside a 16-row pass give identical bits.
+// stream. Passes of up to 16 rows all run on the row kernels, where a row's arithmetic does not depend
+// on the rows beside it: a row decoded alone and inside a 16-row pass give identical bits. A
+// prompt chunk's K slices and attention shape follow its number of rows.
 //
 // Every kernel reads the position and the stop flag from the device State, so a decode
 // step recorded in a hipGraph replays correctly.
@@ -25,9 +26,9 @@
 #include "ill_plan.h"
 
 // Rows of a prompt chunk at most (less where the context is shorter). The GEMMs need many rows
-// to fill the chip: whole prompts in chunks of 512 / 1024 / 2048 rows took 16.9 / 13.6 / 11.6 ms
-// (f16, 4000 tokens), 7.6 / 6.0 / 5.0 (2000), 3.2 / 2.3 / 2.3 (700); q4 18.7 / 15.0 / 12.7 (4000).
-// The activations of 4096 rows take 90 MB.
+// to fill the chip: whole prompts in chunks of 1280 / 2048 / 4096 rows, ms: 4000 tokens q4 11.7 / 8.7 /
+// 7.1, q8 11.7 / 9.2 / 7.4, f16 11.2 / 8.7 / 7.2; 3000 tokens q4 8.3 / 7.0 / 5.6; 2500 tokens q4
+// 6.0 / 6.1 / 4.9. The activations of 4096 rows take 90 MB.
 #define ILL_OP_MAXM 4096
 
 struct OpMat {
@@ -130,8 +131,6 @@ __device__ __forceinline__ float op_dequant1(const OpMat& m, int r, int k) {
   }
 }
 
-// x[t][:] = embedding row of ptoks[t] (Shaders.swift:118-126, :179-190)
-
 // xn[t] = f16(x[t] * rsqrt(mean(x^2) + eps) * gamma) for rows row0 .. row0 + M - 1 (one wave
 // per row; sum of squares in a fixed order). Output row index t - row0.
 __global__ __launch_bounds__(256) void op_norm_kernel(OpCtx c, const float* gamma, int row0, int M) {
@@ -157,7 +156,7 @@ __global__ __launch_bounds__(256) void op_norm_kernel(OpCtx c, const float* gamm
     gst((uint16_t*)(c.xn + (size_t)t * ILL_H + 64 * i + lane), (uint16_t)__half_as_ushort(__float2half(v[i] * scale * g[i])));
 }
 
-// The embedding rows of the pass's tokens into x and, from the same registers, layer 0's
+// The embedding rows of the pass's tokens (Shaders.swift:118-126, :179-190) into x and, from the same registers, layer 0's
 // RMSNorm of them into xn, in one launch (one wave per row; the sum of squares in
 // op_norm_kernel's order).
 template <int FMT>
@@ -415,12 +414,13 @@ __device__ __forceinline__ OpTile op_tile_xcd() {
 //   A: BM rows x 64 halves, row by row, the 8 16-byte units of a row permuted (k / 8 at place
 //      k / 8 ^ row / 2 % 8): eight lanes of a load take a row's whole 128-byte line, and the 16 lanes
 //      of an operand read (16 rows) fall on different banks. (Units ordered (row / 16, k / 8,
-//      row % 16) read without conflicts too, but the loads gathered 16 bytes of 16 rows: AOLD);
+//      row % 16) read without conflicts too, but each load gathered 16 bytes of 64 places: gate/up,
+//      f16, 66 us against 53 at 2000 rows);
 //   B: the k-step's block of the tiled weights (128 rows x 64 columns at op_wt_off, 4 KB q4,
 //      8 KB q8, 16 KB f16) as stored: its units are already in that order;
 //   q8: the block's scales (128 rows x 64 / qg f16, op_st_off), 256 or 512 bytes.
-// q8 and q4 weights are dequantized as they leave LDS. The loads are issued in inline assembly: the compiler's own tracking of LDS
-// loads in flight made it wait for all of them before some of the stage's LDS reads (it
+// q8 and q4 weights are dequantized as they leave LDS. The loads are issued in inline assembly: the
+// compiler's own tracking of LDS loads in flight made it wait for all of them before some of the stage's LDS reads (it
 // could not tell the stages apart), which serialized the ring. The wait for the stage about
 // to be read is explicit: vmcnt counts this wave's own loads, and the barrier after it covers
 // the other waves' loads and orders every wave's reads of the stage refilled next before the
@@ -537,11 +537,7 @@ __device__ __forceinline__ void op_ring_wait(int later) {
   switch (later) {
     case 0: op_vm_barrier<0>(); break;
     case 1: op_vm_barrier<L>(); break;
-    case 2: op_vm_barrier<2 * L>(); break;
-    case 3: op_vm_barrier<3 * L>(); break;
-    case 4: op_vm_barrier<4 * L>(); break;
-    case 5: op_vm_barrier<5 * L>(); break;
-    default: op_vm_barrier<6 * L>(); break;
+    default: op_vm_barrier<2 * L>(); break;
   }
 }
 
@@ -549,16 +545,14 @@ __device__ __forceinline__ void op_ring_wait(int later) {
 // the 128-column tile and all BM rows).
 template <int FMT, int BM, int EPI, int ST>
 __global__ __launch_bounds__(256, EPI == OP_SILU ? 3 : 2) void op_gemm_ring_kernel(OpGemmArgs a) {
-  static_assert(ST >= 2 && ST <= 8 && BM >= 16 && BM <= 64 && (EPI != OP_LMH || BM == 16), "ring GEMM shape");
+  static_assert(ST >= 2 && ST <= 4 && BM >= 16 && BM <= 64 && (EPI != OP_LMH || BM == 16), "ring GEMM shape");
   using R = OpRing<FMT, BM>;
   const OpHdr hd = op_hdr(a.c);
 #define OP_RING_ARR(i) __shared__ __attribute__((aligned(16))) uint4 r##i[ST > i ? R::N : 1];
-  OP_RING_ARR(0) OP_RING_ARR(1) OP_RING_ARR(2) OP_RING_ARR(3) OP_RING_ARR(4) OP_RING_ARR(5) OP_RING_ARR(6) OP_RING_ARR(7)
+  OP_RING_ARR(0) OP_RING_ARR(1) OP_RING_ARR(2) OP_RING_ARR(3)
 #undef OP_RING_ARR
   __shared__ uint64_t red[4][16];   // (the argmax epilogue only)
-  auto ring = [&](int d) -> uint4* {
-    return d == 0 ? r0 : d == 1 ? r1 : d == 2 ? r2 : d == 3 ? r3 : d == 4 ? r4 : d == 5 ? r5 : d == 6 ? r6 : r7;
-  };
+  auto ring = [&](int d) -> uint4* { return d == 0 ? r0 : d == 1 ? r1 : d == 2 ? r2 : r3; };
   constexpr int TM = BM / 16;
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
   const int kg = lane >> 4, n = lane & 15;
@@ -618,13 +612,11 @@ __global__ __launch_bounds__(256, EPI == OP_SILU ? 3 : 2) void op_gemm_ring_kern
   }
 }
 
-// Residual split-K reduction fused with the RMSNorm that reads the updated residual, for
-// passes of up to 16 rows: one workgroup per row m, one thread per column. x[m] += the
-// slices' partials (added in slice order); then, for rows m >= row0,
-// xn[m - row0] = f16(x * rsqrt(mean(x^2) + eps) * gamma), the sum of squares taken per wave
-// and the 14 wave sums added in order (a function of the row alone, so 1-row and 16-row
-// passes agree bit for bit).
-__global__ __launch_bounds__(ILL_H) void op_epi_norm_kernel(OpGemmArgs a, int S, const float* gamma, int row0) {
+// Residual split-K reduction of a prompt chunk fused with the RMSNorm that reads the updated
+// residual: one workgroup per row m, one thread per column. x[m] += the slices' partials (added in
+// slice order), xn[m] = f16(x * rsqrt(mean(x^2) + eps) * gamma), the sum of squares taken per wave
+// and the 14 wave sums added in order.
+__global__ __launch_bounds__(ILL_H) void op_epi_norm_kernel(OpGemmArgs a, int S, const float* gamma) {
   __shared__ float red[ILL_H / 64];
   const OpHdr hd = op_hdr(a.c);
   const int m = blockIdx.x, j = threadIdx.x, w = j >> 6, lane = j & 63;
@@ -639,7 +631,6 @@ __global__ __launch_bounds__(ILL_H) void op_epi_norm_kernel(OpGemmArgs a, int S,
     if (z < S) y += pz[z];
   const float v = gld(r) + y;
   if (!hd.done) gst(r, v);
-  if (m < row0) return;   // the whole workgroup
   const float ss = gsum<64>(v * v);
   if (lane == 0) red[w] = ss;
   __syncthreads();
@@ -648,7 +639,7 @@ __global__ __launch_bounds__(ILL_H) void op_epi_norm_kernel(OpGemmArgs a, int S,
   for (int i = 0; i < ILL_H / 64; i++) tot += red[i];
   const float scale = __builtin_amdgcn_rsqf(tot * (1.0f / (float)ILL_H) + ILL_EPS);
   if (hd.done) return;
-  gst((uint16_t*)(a.c.xn + (size_t)(m - row0) * ILL_H + j), (uint16_t)__half_as_ushort(__float2half(v * scale * g)));
+  gst((uint16_t*)(a.c.xn + (size_t)m * ILL_H + j), (uint16_t)__half_as_ushort(__float2half(v * scale * g)));
 }
 
 // (m, l, o) of n states combined against their maximum, in index order; states with

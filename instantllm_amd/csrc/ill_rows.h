@@ -16,10 +16,10 @@
 //
 // Measured against one kernel more per layer, with the gate/up and down products' K-slice
 // partials in memory, the O projection inside attention and the residual sums and norms in
-// kernels of their own (graph-replayed steps, us): q8 852 -> 584 after 512 positions, 970 ->
-// 599 at 4000; f16 850 -> 644 and 969 -> 661; passes of 4 rows at 512 positions q8 950 -> 650,
-// of 16 rows 1,230 -> 1,103. Kernel times of a q8 step at 512 positions: QKV 3.7, attention
-// 6.4, O 3.6, gate/up 4.4, down 4.7 us.
+// kernels of their own (graph-replayed steps, us): q8 852 -> 591 after 512 positions, 970 ->
+// 606 at 4000; f16 850 -> 656 and 969 -> 672; passes of 16 rows after 500 positions, q8, host
+// clock, 1,294 -> 944. Kernel times of a q8 step at 512 positions: QKV 3.8, attention 6.8, O 3.8,
+// gate/up 4.5, down 4.7 us.
 //
 // A row's arithmetic does not depend on the rows beside it or on MT (rows a workgroup holds):
 // every output is the same MFMA sequence over K in the same order, and the attention's
