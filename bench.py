@@ -49,16 +49,16 @@ KV_BYTES_PER_POS = 12_288         # 24 layers x 2 KV heads x (K + V) x 64 x 2 B
 # Source and commands: profiles/pass_kernel_q4_decode_config2.md
 TRAFFIC_BYTES_PER_STEP = 349_899_200
 # MFMA utilisation of the pass kernels (commit 12e9d07) and of the prefill kernels (commit
-# fdc1ab0), from rocprofv3 SQ_VALU_MFMA_BUSY_CYCLES over the kernel durations
+# 89bb7e2), from rocprofv3 SQ_VALU_MFMA_BUSY_CYCLES over the kernel durations
 # (profiles/pass_kernel_q4_decode_config2.md, profiles/layer_by_layer_q8_f16_config4.md)
 MFMA_COUNTERS = {
     "ill_pass_kernel<16> (16-row verify)": {"mfma_busy": 0.0111, "int8_TOPs": 48.1},
     "ill_pass_kernel<1> (1-row step)": {"mfma_busy": 0.0122, "int8_TOPs": 54.8},
-    "prefill gate/up GEMM (f16, 512 rows)": {"mfma_busy": 0.201, "f16_TFLOPs": 505},
-    "prefill O GEMM (f16, 512 rows)": {"mfma_busy": 0.050, "f16_TFLOPs": 125},
-    "prefill down GEMM (f16, 512 rows)": {"mfma_busy": 0.144, "f16_TFLOPs": 361},
-    "prefill QKV GEMM (f16, 512 rows)": {"mfma_busy": 0.038, "f16_TFLOPs": 96},
-    "prefill attention (512 rows, q8 / f16)": {"mfma_busy": 0.058, "f16_TFLOPs": 145},
+    "prefill gate/up GEMM (f16, 512 rows)": {"mfma_busy": 0.184, "f16_TFLOPs": 463},
+    "prefill O GEMM (f16, 512 rows)": {"mfma_busy": 0.048, "f16_TFLOPs": 120},
+    "prefill down GEMM (f16, 512 rows)": {"mfma_busy": 0.143, "f16_TFLOPs": 359},
+    "prefill QKV GEMM (f16, 512 rows)": {"mfma_busy": 0.039, "f16_TFLOPs": 97},
+    "prefill attention (512 rows, q8 / f16)": {"mfma_busy": 0.058, "f16_TFLOPs": 146},
 }
 
 
